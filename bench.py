@@ -451,8 +451,7 @@ def bench_adjoint(args, lqcd):
     t_fb_dev = time.perf_counter() - t0
     del gbuf
     integ = lqcd.SymplecticEulerGpu(lqcd.DRIFT_ADDITIVE, lqcd.SCHEME_REFERENCE)
-    # kernel times from profiled trajectories on a copy of the state (with
-    # profiling on, the reference scheme launches eagerly, not from a graph)
+    # kernel times from profiled trajectories on a copy of the state
     prof = lqcd.LatticeStateDefault(st.lattice(), beta, st.link_matrix(), lqcd.F64)
     hmc_p = lqcd.HybridMonteCarloDiagnostic(dt, md, integ, args.seed + 1, project_gauss=False)
     pctx = prof._dev.ctx
@@ -938,8 +937,7 @@ def bench_small(args, lqcd):
     ctx = st._dev.ctx
     hmc.next_element(st)
     mh.next_element(st)
-    # kernel times from two profiled trajectories on a copy of the state (with
-    # profiling on the reference scheme launches eagerly, not from a graph)
+    # kernel times from two profiled trajectories on a copy of the state
     prof = lqcd.LatticeStateDefault(st.lattice(), beta, st.link_matrix(), lqcd.F64)
     hmc_p = lqcd.HybridMonteCarloDiagnostic(dt, md, lqcd.SymplecticEulerGpu(lqcd.DRIFT_ADDITIVE,
                                                                           lqcd.SCHEME_REFERENCE), args.seed + 1,

@@ -63,8 +63,9 @@ typedef enum { LQCD_F64 = 0, LQCD_F32 = 1 } lqcd_precision;
 typedef enum { LQCD_DRIFT_ADDITIVE = 0, LQCD_DRIFT_EXP = 1 } lqcd_drift;
 
 /* REFERENCE = n calls of integrate_symplectic, kick(dt/2) drift(dt)
- * kick(dt/2) each (symplectic_euler_rayon.rs:222-252); LEAPFROG merges the
- * two half kicks between consecutive steps (n + 1 force evaluations), which
+ * kick(dt/2) each (symplectic_euler_rayon.rs:222-252), the two half
+ * kicks that meet between steps applied one after the other with one force;
+ * LEAPFROG merges them into one kick, which
  * is simulate_using_leapfrog_n (src/simulation/state.rs:321-358). */
 typedef enum { LQCD_SCHEME_REFERENCE = 0, LQCD_SCHEME_LEAPFROG = 1 } lqcd_scheme;
 
@@ -368,8 +369,8 @@ int lqcd_md_variant_get(const lqcd_lattice* lat, int* variant);
  * integration or device Metropolis sweep read two rows. */
 int lqcd_md_reconstruct_set(lqcd_lattice* lat, int mode);
 /* 1 (default): the MD launches of an integration are replayed from a HIP
- * graph captured on first use for the starting buffer and parameters (the
- * reference scheme only while profiling is off); 0: launched one by one.
+ * graph captured on first use for the starting buffer and parameters;
+ * 0: launched one by one.
  * Same results; the graph removes the ~10 us the device leaves between eager
  * launches.  No counterpart in the reference. */
 int lqcd_md_graph_set(lqcd_lattice* lat, int enable);

@@ -87,8 +87,9 @@ struct lqcd_batch {
 namespace lqcd {
 
 // ---- batched kernels (k_batch.hip); all on b->ctx->stream ----
+// (twice: the kick applied twice with one force, kick_link in md_device.hpp)
 hipError_t launch_batch_md(const lqcd_batch* b, int config, const void* U_in, void* U_out, double kick,
-                           double dt, int op);
+                           double dt, int op, bool twice = false);
 // settles the grid of launch_batch_md(config, op) without launching
 hipError_t prepare_batch_md(const lqcd_batch* b, int config, int op);
 hipError_t launch_batch_momenta(const lqcd_batch* b);

@@ -69,21 +69,16 @@ hipError_t batch_integrate(const lqcd_batch* b, int config, double dt, size_t n,
 {
     int src = 0, dst = 1;
     hipError_t e = hipSuccess;
-    if (scheme == LQCD_SCHEME_REFERENCE) {
-        for (size_t k = 0; k < n && e == hipSuccess; ++k) {
-            e = launch_batch_md(b, config, b->U[src], b->U[dst], dt / 2.0, dt, drift);
-            if (e == hipSuccess) e = launch_batch_md(b, config, b->U[dst], nullptr, dt / 2.0, dt, BATCH_KICK);
-            src = dst;
-            dst = dst == 1 ? 2 : 1;
-        }
-    } else {
-        for (size_t k = 0; k < n && e == hipSuccess; ++k) {
-            e = launch_batch_md(b, config, b->U[src], b->U[dst], k == 0 ? dt / 2.0 : dt, dt, drift);
-            src = dst;
-            dst = dst == 1 ? 2 : 1;
-        }
-        if (e == hipSuccess) e = launch_batch_md(b, config, b->U[src], nullptr, dt / 2.0, dt, BATCH_KICK);
+    // as integrate_steps (capi.cpp): the kicks of dt/2 that end a step of the
+    // reference scheme and start the next are one launch's two kicks
+    const bool ref = scheme == LQCD_SCHEME_REFERENCE;
+    for (size_t k = 0; k < n && e == hipSuccess; ++k) {
+        const double kick = k == 0 || ref ? dt / 2.0 : dt;
+        e = launch_batch_md(b, config, b->U[src], b->U[dst], kick, dt, drift, k > 0 && ref);
+        src = dst;
+        dst = dst == 1 ? 2 : 1;
     }
+    if (e == hipSuccess) e = launch_batch_md(b, config, b->U[src], nullptr, dt / 2.0, dt, BATCH_KICK);
     *last = src;
     return e;
 }

@@ -143,9 +143,9 @@ enum MdVariant {
 // VAR_SITE_TILE's LDS tile: whether it applies to the lattice, and its bytes
 bool md_tile_fits(const lqcd_lattice* L);
 size_t md_tile_bytes(const lqcd_lattice* L);
-// What an MD launch of the per-site kernels (variants 2-4) does besides its
-// kick (+ drift): sums (MdSums in md_device.hpp: 0 none, 1 before the kick,
-// 2 after it) of Re Tr(U Sigma) and e^2 into partials[block][0..1] (a
+// What an MD launch does besides its kick (+ drift).  Every variant: sums 3
+// (MdSums in md_device.hpp), the kick applied twice.  The per-site kernels
+// (variants 2-4): sums (0 none, 1 before the kick, 2 after it) of Re Tr(U Sigma) and e^2 into partials[block][0..1] (a
 // workgroup per 256 sites), and with two-row reads row 2 of the links read
 // written to row2 (null: not).
 struct MdExtra {

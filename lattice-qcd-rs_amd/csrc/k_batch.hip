@@ -25,7 +25,8 @@ constexpr uint32_t kAcceptBlock = 62;
 // MD over all chains.  Work units are tiles (SITE) or (tile, mu) pairs, mu
 // fastest; workgroup wg (XCD-remapped) owns the contiguous unit range
 // [wg * chunk, (wg + 1) * chunk) and its waves take every W-th unit of it.
-template <int D, typename S, int DR, bool SITE, bool R12>
+// TWICE: two kicks per launch (kick_link).
+template <int D, typename S, int DR, bool SITE, bool R12, bool TWICE>
 __global__ __launch_bounds__(kBlock) void k_batch_md(const vec2_t<S>* __restrict__ U_in,
                                                      vec2_t<S>* __restrict__ U_out, S* __restrict__ E,
                                                      const ChainDesc* __restrict__ cd,
@@ -54,9 +55,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_md(const vec2_t<S>* __restrict
         // trajectory rebuilds row 2 of its final links, k_batch_links_map<2>)
         constexpr bool R01 = R12 && DR == DRIFT_EXP;
         if (SITE)
-            md_site<D, S, S, DR, R12, false, R01>(ui, uo, e, d.g, s, fs, (S)kick, df);
+            md_site<D, S, S, DR, R12, false, R01, TWICE ? KICK_TWICE : SUMS_NONE>(ui, uo, e, d.g, s, fs, (S)kick, df);
         else
-            md_link<D, S, S, DR, R12, R01>(ui, uo, e, d.g, mu, s, fs, (S)kick, df);
+            md_link<D, S, S, DR, R12, R01, TWICE>(ui, uo, e, d.g, mu, s, fs, (S)kick, df);
     }
 }
 
@@ -309,7 +310,7 @@ static int64_t resident_blocks(K kernel, int block)
 
 // launch == false only settles the grid (the occupancy query), so that a
 // later launch under stream capture makes no device query
-template <int D, typename S, int DR, bool SITE, bool R12>
+template <int D, typename S, int DR, bool SITE, bool R12, bool TWICE>
 static hipError_t batch_md(const lqcd_batch* b, int block, bool persistent, const void* U_in, void* U_out,
                            double kick, double dt, bool launch)
 {
@@ -319,18 +320,18 @@ static hipError_t batch_md(const lqcd_batch* b, int block, bool persistent, cons
     if (persistent) {
         static int64_t resident[5] = {-1, -1, -1, -1, -1};  // by block / 64
         int64_t& res = resident[W];
-        if (res < 0) res = resident_blocks(k_batch_md<D, S, DR, SITE, R12>, block);
+        if (res < 0) res = resident_blocks(k_batch_md<D, S, DR, SITE, R12, TWICE>, block);
         if (res > 0 && res < groups) groups = res;
     }
     if (!launch) return hipSuccess;
     const int64_t chunk = (nunit + groups - 1) / groups;
-    k_batch_md<D, S, DR, SITE, R12><<<(unsigned)groups, block, 0, b->ctx->stream>>>(
+    k_batch_md<D, S, DR, SITE, R12, TWICE><<<(unsigned)groups, block, 0, b->ctx->stream>>>(
         (const vec2_t<S>*)U_in, (vec2_t<S>*)U_out, (S*)b->E, b->d_chains, b->d_tile_chain, nunit, chunk,
         kick, dt);
     return hipGetLastError();
 }
 
-template <int D, typename S, int DR>
+template <int D, typename S, int DR, bool TWICE>
 static hipError_t batch_md_shape(const lqcd_batch* b, int config, const void* U_in, void* U_out, double kick,
                                  double dt, bool launch)
 {
@@ -339,41 +340,46 @@ static hipError_t batch_md_shape(const lqcd_batch* b, int config, const void* U_
     if constexpr (DR != DRIFT_ADDITIVE) {
         if (b->md_r12) {
             if (sh.site)
-                return batch_md<D, S, DR, true, true>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
-            return batch_md<D, S, DR, false, true>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
+                return batch_md<D, S, DR, true, true, TWICE>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
+            return batch_md<D, S, DR, false, true, TWICE>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
         }
     }
-    if (sh.site) return batch_md<D, S, DR, true, false>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
-    return batch_md<D, S, DR, false, false>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
+    if (sh.site) return batch_md<D, S, DR, true, false, TWICE>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
+    return batch_md<D, S, DR, false, false, TWICE>(b, sh.block, sh.persistent, U_in, U_out, kick, dt, launch);
 }
 
 static hipError_t batch_md_op(const lqcd_batch* b, int config, const void* U_in, void* U_out, double kick,
-                              double dt, int op, bool launch)
+                              double dt, int op, bool launch, bool twice)
 {
     if (config < 0 || config >= kBatchConfigs) return hipErrorInvalidValue;
     if (op == BATCH_KICK) {
-        BATCH_DISPATCH(b, return (batch_md_shape<D, S, -1>(b, config, U_in, U_out, kick, dt, launch)));
+        BATCH_DISPATCH(b, return (batch_md_shape<D, S, -1, false>(b, config, U_in, U_out, kick, dt, launch)));
     } else if (op == DRIFT_EXP) {
-        BATCH_DISPATCH(b, return (batch_md_shape<D, S, DRIFT_EXP>(b, config, U_in, U_out, kick, dt, launch)));
+        if (twice)
+            BATCH_DISPATCH(b, return (batch_md_shape<D, S, DRIFT_EXP, true>(b, config, U_in, U_out, kick, dt, launch)));
+        BATCH_DISPATCH(b, return (batch_md_shape<D, S, DRIFT_EXP, false>(b, config, U_in, U_out, kick, dt, launch)));
     } else {
-        BATCH_DISPATCH(b, return (batch_md_shape<D, S, DRIFT_ADDITIVE>(b, config, U_in, U_out, kick, dt, launch)));
+        if (twice)
+            BATCH_DISPATCH(b, return (batch_md_shape<D, S, DRIFT_ADDITIVE, true>(b, config, U_in, U_out, kick, dt, launch)));
+        BATCH_DISPATCH(b, return (batch_md_shape<D, S, DRIFT_ADDITIVE, false>(b, config, U_in, U_out, kick, dt, launch)));
     }
     return hipErrorInvalidValue;
 }
 
 hipError_t launch_batch_md(const lqcd_batch* b, int config, const void* U_in, void* U_out, double kick,
-                           double dt, int op)
+                           double dt, int op, bool twice)
 {
     lqcd_prof_event ev;
     prof_begin(b->ctx, op == BATCH_KICK ? PROF_KICK : PROF_KICK_DRIFT, &ev);
-    const hipError_t e = batch_md_op(b, config, U_in, U_out, kick, dt, op, true);
+    const hipError_t e = batch_md_op(b, config, U_in, U_out, kick, dt, op, true, twice);
     prof_end(b->ctx, &ev);
     return e;
 }
 
 hipError_t prepare_batch_md(const lqcd_batch* b, int config, int op)
 {
-    return batch_md_op(b, config, nullptr, nullptr, 0.0, 0.0, op, false);
+    const hipError_t e = batch_md_op(b, config, nullptr, nullptr, 0.0, 0.0, op, false, false);
+    return e == hipSuccess ? batch_md_op(b, config, nullptr, nullptr, 0.0, 0.0, op, false, true) : e;
 }
 
 hipError_t launch_batch_momenta(const lqcd_batch* b)

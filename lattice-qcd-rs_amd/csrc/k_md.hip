@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kBlock) void k_derivative_u(const vec2_t<S>* __rest
 }
 
 // VAR_LINK: grid (site blocks, D)
-template <int D, typename S, typename T, int DR, bool R12>
+template <int D, typename S, typename T, int DR, bool R12, bool TWICE>
 __global__ __launch_bounds__(kBlock) void k_md_link(const vec2_t<S>* __restrict__ U_in,
                                                     vec2_t<S>* __restrict__ U_out,
                                                     S* __restrict__ E, Geom g, T fscale, T kick,
@@ -115,11 +115,11 @@ __global__ __launch_bounds__(kBlock) void k_md_link(const vec2_t<S>* __restrict_
     const int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int mu = blockIdx.y;
     if (s >= g.nsite) return;
-    md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP>(U_in, U_out, E, g, mu, s, fscale, kick, dfac);
+    md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP, TWICE>(U_in, U_out, E, g, mu, s, fscale, kick, dfac);
 }
 
 // VAR_LINK_XCD: 1-D grid of (site block, mu) pairs, mu fastest, XCD remapped
-template <int D, typename S, typename T, int DR, bool R12>
+template <int D, typename S, typename T, int DR, bool R12, bool TWICE>
 __global__ __launch_bounds__(kBlock) void k_md_link_xcd(const vec2_t<S>* __restrict__ U_in,
                                                         vec2_t<S>* __restrict__ U_out,
                                                         S* __restrict__ E, Geom g, T fscale, T kick,
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kBlock) void k_md_link_xcd(const vec2_t<S>* __restr
     const int mu = (int)(logical % D);
     const int64_t s = (logical / D) * kBlock + threadIdx.x;
     if (s >= g.nsite) return;
-    md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP>(U_in, U_out, E, g, mu, s, fscale, kick, dfac);
+    md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP, TWICE>(U_in, U_out, E, g, mu, s, fscale, kick, dfac);
 }
 
 // VAR_SITE_XCD / VAR_SITE_SLAB (slab_p > 0): one thread per site, all D links.
@@ -151,9 +151,9 @@ void k_md_site_xcd(const vec2_t<S>* __restrict__ U_in,
     constexpr bool OWN = R12 && sizeof(T) == 4;
     __shared__ vec2_t<T> own_lds[OWN ? D * 9 * kBlock : 1];
     constexpr bool R01 = R12 && DR == DRIFT_EXP;
-    if constexpr (SUMS == SUMS_NONE) {
+    if constexpr (!md_sums(SUMS)) {
         if (s >= g.nsite) return;
-        md_site<D, S, T, DR, R12, OWN, R01>(U_in, U_out, E, g, s, fscale, kick, dfac, own_lds, nullptr, row2);
+        md_site<D, S, T, DR, R12, OWN, R01, SUMS>(U_in, U_out, E, g, s, fscale, kick, dfac, own_lds, nullptr, row2);
     } else {
         MdAcc<T> acc;
         if (s < g.nsite)
@@ -232,7 +232,7 @@ void k_md_site_tile(const vec2_t<S>* __restrict__ U_in,
             mat3<T> m;
             mul<false, false>(u, sig[mu], m);
             im_trace_combinations(m, f[mu]);
-            if constexpr (SUMS != SUMS_NONE) acc.tr += re_trace(m);
+            if constexpr (md_sums(SUMS)) acc.tr += re_trace(m);
         }
     }
     T e[D][8];
@@ -240,7 +240,7 @@ void k_md_site_tile(const vec2_t<S>* __restrict__ U_in,
     for (int mu = 0; mu < D; ++mu) {
         load_e<T, S, kCacheStream>(E, g.npad, mu, s, e[mu]);
         if constexpr (SUMS == SUMS_BEFORE_KICK) acc.e2 += e_squares8<T>(e[mu]);
-        kick_generators(f[mu], kick * fscale, e[mu]);
+        kick_link<SUMS == KICK_TWICE>(f[mu], fscale, kick, e[mu]);
         if constexpr (SUMS == SUMS_AFTER_KICK) acc.e2 += e_squares8<T>(e[mu]);
         store_e<T, S, kCacheStream>(E, g.npad, mu, s, e[mu]);
     }
@@ -255,7 +255,7 @@ void k_md_site_tile(const vec2_t<S>* __restrict__ U_in,
             drift_store<DR, DR == DRIFT_EXP, S, T>(u, e[mu], dfac, U_out, g, mu, s);
         }
     }
-    if constexpr (SUMS != SUMS_NONE) {
+    if constexpr (md_sums(SUMS)) {
         double v[2] = {(double)acc.tr, (double)acc.e2};
         block_reduce_to<2>(v, partials + (int64_t)blockIdx.x * kReduceSlots);
     }
@@ -335,6 +335,7 @@ static void launch_md_variant_r(const lqcd_lattice* L, int variant, const void* 
     hipStream_t st = L->ctx->stream;
     const unsigned nsb = grid_for(L->g.nsite);
     const int sums = x ? x->sums : SUMS_NONE;
+    const bool twice = DR >= 0 && sums == KICK_TWICE;
     switch (variant) {
     case VAR_SITE_TILE:
     case VAR_SITE_XCD:
@@ -348,17 +349,26 @@ static void launch_md_variant_r(const lqcd_lattice* L, int variant, const void* 
             slab_g = Ls / 8;
         }
         constexpr int SUMS_ON = DR >= 0 ? SUMS_BEFORE_KICK : SUMS_AFTER_KICK;
-        if (sums == SUMS_NONE)
+        if (twice)
+            launch_site<D, S, DR, R12, DR >= 0 ? KICK_TWICE : SUMS_NONE>(L, tile, nsb, ui, uo, e, fs, k, df, slab_p,
+                                                                         slab_g, x);
+        else if (sums == SUMS_NONE)
             launch_site<D, S, DR, R12, SUMS_NONE>(L, tile, nsb, ui, uo, e, fs, k, df, slab_p, slab_g, x);
         else
             launch_site<D, S, DR, R12, SUMS_ON>(L, tile, nsb, ui, uo, e, fs, k, df, slab_p, slab_g, x);
         break;
     }
     case VAR_LINK_XCD:
-        k_md_link_xcd<D, S, S, DR, R12><<<nsb * (unsigned)D, kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
+        if (twice)
+            k_md_link_xcd<D, S, S, DR, R12, DR >= 0><<<nsb * (unsigned)D, kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
+        else
+            k_md_link_xcd<D, S, S, DR, R12, false><<<nsb * (unsigned)D, kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
         break;
     default:
-        k_md_link<D, S, S, DR, R12><<<link_grid(L), kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
+        if (twice)
+            k_md_link<D, S, S, DR, R12, DR >= 0><<<link_grid(L), kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
+        else
+            k_md_link<D, S, S, DR, R12, false><<<link_grid(L), kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
         break;
     }
 }

@@ -347,8 +347,22 @@ __device__ __forceinline__ void drift_store(const mat3<T>& u, const T* e, T dfac
     }
 }
 
+// The momentum kick of one link from its generator combinations.  TWICE: a
+// second kick by the same force, applied after the first with a rounding of
+// its own.  The reference scheme ends a step with a kick of dt/2 and starts the
+// next with another at the same links; forming the force once for the pair
+// gives the same bits as a launch for each (the force does not depend on E).
+// A template flag, as a branch here splits the block that the scheduler works
+// on: with `if (kick2 != 0)` the per-site kernels spilled 1.2-4.9 KB per lane.
+template <bool TWICE, typename T>
+__device__ __forceinline__ void kick_link(const T* f, T fscale, T kick, T* e)
+{
+    kick_generators(f, kick * fscale, e);
+    if constexpr (TWICE) kick_generators(f, kick * fscale, e);
+}
+
 // what happens with the force of one link (DR: -1 kick only, else drift mode)
-template <int DR, typename S, typename T, bool R01 = false>
+template <int DR, typename S, typename T, bool R01 = false, bool TWICE = false>
 __device__ __forceinline__ void finish_link(const mat3<T>& u, const mat3<T>& sigma,
                                             vec2_t<S>* __restrict__ U_out, S* __restrict__ E,
                                             const Geom& g, int mu, int64_t s, T fscale, T kick,
@@ -359,15 +373,16 @@ __device__ __forceinline__ void finish_link(const mat3<T>& u, const mat3<T>& sig
     T f[8], e[8];
     im_trace_combinations(m, f);
     load_e<T, S, kCacheStream>(E, g.npad, mu, s, e);
-    kick_generators(f, kick * fscale, e);
+    kick_link<TWICE>(f, fscale, kick, e);
     store_e<T, S, kCacheStream>(E, g.npad, mu, s, e);
     if constexpr (DR >= 0) drift_store<DR, R01, S, T>(u, e, dfac, U_out, g, mu, s);
 }
 
-// one link (mu, s): e += kick * F(U_in); U_out = drift(U_in, e) unless DR < 0.
+// one link (mu, s): e += kick * F(U_in) (TWICE: two such kicks); U_out =
+// drift(U_in, e) unless DR < 0.
 // R12: links read as two rows (load_link_r12), for links in SU(3); R01: the
 // drifted link is stored as rows 0, 1 only.
-template <int D, typename S, typename T, int DR, bool R12 = false, bool R01 = false>
+template <int D, typename S, typename T, int DR, bool R12 = false, bool R01 = false, bool TWICE = false>
 __device__ __forceinline__ void md_link(const vec2_t<S>* __restrict__ U_in, vec2_t<S>* __restrict__ U_out,
                                         S* __restrict__ E, const Geom& g, int mu, int64_t s, T fscale,
                                         T kick, T dfac)
@@ -376,7 +391,7 @@ __device__ __forceinline__ void md_link(const vec2_t<S>* __restrict__ U_in, vec2
     mat3<T> sigma;
     staple_sum<D, S, T, R12>(U_in, g, mu, s, nb, sigma);
     const mat3<T> u = load_link_sel<R12, T, S>(U_in, g.npad, mu, s);
-    finish_link<DR, S, T, R01>(u, sigma, U_out, E, g, mu, s, fscale, kick, dfac);
+    finish_link<DR, S, T, R01, TWICE>(u, sigma, U_out, E, g, mu, s, fscale, kick, dfac);
 }
 
 // The Hamiltonian sums a fused MD launch can produce on the way (SUMS): the
@@ -385,7 +400,9 @@ __device__ __forceinline__ void md_link(const vec2_t<S>* __restrict__ U_in, vec2
 // and the momentum sum sum_mu,a e^a_mu(x)^2 of E before the kick
 // (SUMS_BEFORE_KICK: the first launch of a trajectory, H_old) or after it
 // (SUMS_AFTER_KICK: the final kick, H_new); accumulated per thread in double.
-enum MdSums { SUMS_NONE = 0, SUMS_BEFORE_KICK = 1, SUMS_AFTER_KICK = 2 };
+// KICK_TWICE is the fourth form of a launch: no sums, two kicks (kick_link).
+enum MdSums { SUMS_NONE = 0, SUMS_BEFORE_KICK = 1, SUMS_AFTER_KICK = 2, KICK_TWICE = 3 };
+__host__ __device__ constexpr bool md_sums(int form) { return form == SUMS_BEFORE_KICK || form == SUMS_AFTER_KICK; }
 template <typename T>
 struct MdAcc {
     T tr = T(0);
@@ -441,14 +458,14 @@ __device__ __forceinline__ void md_site(const vec2_t<S>* __restrict__ U_in, vec2
             mat3<T> m;
             mul<false, false>(u, sig[mu], m);
             im_trace_combinations(m, f[mu]);
-            if constexpr (SUMS != SUMS_NONE) acc->tr += re_trace(m);
+            if constexpr (md_sums(SUMS)) acc->tr += re_trace(m);
         }
     }
     // phase 2: momentum kicks of the D links
 #pragma unroll
     for (int mu = 0; mu < D; ++mu) {
         if constexpr (SUMS == SUMS_BEFORE_KICK) acc->e2 += e_squares8<T>(e[mu]);
-        kick_generators(f[mu], kick * fscale, e[mu]);
+        kick_link<SUMS == KICK_TWICE>(f[mu], fscale, kick, e[mu]);
         if constexpr (SUMS == SUMS_AFTER_KICK) acc->e2 += e_squares8<T>(e[mu]);
         store_e<T, S, kCacheStream>(E, g.npad, mu, s, e[mu]);
     }
