@@ -259,10 +259,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_accept_copy(const vec2_t<S>* _
     const ChainDesc& d = cd[c];
     const int64_t s = (tile - d.tile0) * kTile + (threadIdx.x & 63);
     if (s >= d.g.nsite) return;
-    const vec2_t<S>* src = U_final + d.u_off + s;
-    vec2_t<S>* dst = U + d.u_off + s;
 #pragma unroll
-    for (int k = 0; k < D * 9; ++k) dst[(int64_t)k * d.g.npad] = src[(int64_t)k * d.g.npad];
+    for (int mu = 0; mu < D; ++mu)
+        store_link<S, S>(U + d.u_off, d.g.npad, mu, s, load_link<S, S>(U_final + d.u_off, d.g.npad, mu, s));
 }
 
 __global__ void k_batch_counter_advance(uint64_t* __restrict__ counter)

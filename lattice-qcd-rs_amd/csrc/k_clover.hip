@@ -99,16 +99,9 @@ struct AllLinks {
     int64_t npad;
     __device__ __forceinline__ mat3<double> operator()(int d, int64_t y) const
     {
-        using E = vec2_t<S>;
-        const __amdgpu_buffer_rsrc_t r = planes_rsrc(U, npad, 9 * D);
-        const uint32_t plane = (uint32_t)npad * (uint32_t)sizeof(E);
-        const uint32_t off = ((uint32_t)d * 9u * (uint32_t)npad + (uint32_t)y) * (uint32_t)sizeof(E);
         mat3<double> m;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-            const E v = buf_load<E>(r, off, (uint32_t)k * plane);
-            m.e[k] = {double(v.x), double(v.y)};
-        }
+        load_entries<0, 9, double, S, kCacheDefault>(planes_rsrc(U, npad, 9 * D), (uint32_t)d * link_plane<S>(npad, 9),
+                                                     npad, y, m);
         return m;
     }
 };
