@@ -68,6 +68,17 @@ __device__ __forceinline__ int64_t slab_block(int64_t j, int64_t P, int64_t G)
     return (q * G + r % G) * P + r / G;
 }
 
+// P and G of slab_block for workgroups of `block` sites, or 0 where the
+// lattice does not allow the order (whole workgroups per slice of the slowest
+// direction, 8 | its extent).
+inline void slab_shape(const Geom& g, int64_t block, int64_t& P, int64_t& G)
+{
+    const int64_t Ls = g.extent[g.dim - 1], slice = g.nsite / Ls;
+    const bool fits = slice % block == 0 && Ls % 8 == 0;
+    P = fits ? slice / block : 0;
+    G = fits ? Ls / 8 : 0;
+}
+
 template <int D>
 __device__ __forceinline__ int site_parity(const Geom& g, int64_t s)
 {

@@ -554,12 +554,7 @@ __global__ __launch_bounds__(kBlock) void k_overrelax(vec2_t<S>* __restrict__ U,
 static ClassOrder class_order(const lqcd_lattice* L)
 {
     ClassOrder co;
-    const int64_t Ls = L->g.extent[L->g.dim - 1];
-    const int64_t slice = L->g.nsite / Ls;
-    if (slice % (2 * kBlock) == 0 && Ls % 8 == 0) {
-        co.slab_p = slice / (2 * kBlock);
-        co.slab_g = Ls / 8;
-    }
+    slab_shape(L->g, 2 * kBlock, co.slab_p, co.slab_g);
     return co;
 }
 

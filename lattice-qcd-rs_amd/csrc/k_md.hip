@@ -40,16 +40,28 @@ namespace lqcd {
 // values into an LDS image of it (rows of D * 8 + 1 doubles, so that the
 // lanes' 8-byte writes fall into different banks) and the block stores the
 // image as whole 16-byte words, lane after lane.
+//
+// Bound by the neighbour links' latency (f64: one wave per SIMD, 440 VGPRs),
+// so the workgroups run in the MD kernels' order (xcd_remap, and slab_block
+// where the lattice allows it), which keeps neighbour blocks on one XCD.
+// Against storage order, same bits: f64 16^4 46.8 -> 37.0 us, 32^4 626 ->
+// 600, 15x13x11x17 32.9 -> 27.3, D = 3 128^3 745 -> 680; f32 24^4 141 -> 90,
+// 32^4 320 -> 300.  Workgroups of 64 or 256 threads, and f64 capped at two waves
+// per SIMD (spills 744 B; 16^4 70.6 us), were not faster.  Reading two rows of
+// SU(3) links is (16^4 30.6 us), but its error against 64 bits is 7 % (f64)
+// and 1 % (f32) larger, so all nine entries are read.
 constexpr int kForceBlock = 128;
 
 template <int D, typename S, typename T>
 __global__ __launch_bounds__(kForceBlock) void k_force_store(const vec2_t<S>* __restrict__ U, Geom g,
                                                              T fscale, double* __restrict__ out,
-                                                             double oscale)
+                                                             double oscale, int64_t slab_p, int64_t slab_g)
 {
     constexpr int kRow = D * 8 + 1;
     __shared__ double img[kForceBlock * kRow];
-    const int64_t s0 = (int64_t)blockIdx.x * kForceBlock;
+    int64_t logical = xcd_remap(blockIdx.x, gridDim.x);
+    if (slab_p > 0) logical = slab_block(logical, slab_p, slab_g);
+    const int64_t s0 = logical * kForceBlock;
     const int64_t s = s0 + threadIdx.x;
     if (s < g.nsite) {
         const Neighbours<D> nb = neighbours<D>(g, s);
@@ -342,12 +354,7 @@ static void launch_md_variant_r(const lqcd_lattice* L, int variant, const void* 
     case VAR_SITE_SLAB: {
         const bool tile = variant == VAR_SITE_TILE && R12 && sizeof(S) == 4 && md_tile_fits(L);
         int64_t slab_p = 0, slab_g = 0;
-        const int64_t Ls = L->g.extent[D - 1];
-        const int64_t slice = L->g.nsite / Ls;
-        if (variant != VAR_SITE_XCD && slice % kBlock == 0 && Ls % 8 == 0) {
-            slab_p = slice / kBlock;
-            slab_g = Ls / 8;
-        }
+        if (variant != VAR_SITE_XCD) slab_shape(L->g, kBlock, slab_p, slab_g);
         constexpr int SUMS_ON = DR >= 0 ? SUMS_BEFORE_KICK : SUMS_AFTER_KICK;
         if (twice)
             launch_site<D, S, DR, R12, DR >= 0 ? KICK_TWICE : SUMS_NONE>(L, tile, nsb, ui, uo, e, fs, k, df, slab_p,
@@ -404,9 +411,12 @@ hipError_t launch_force_store(const lqcd_lattice* L, const void* U, double* d_ou
 {
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_FORCE_STORE, &ev);
+    int64_t slab_p, slab_g;
+    slab_shape(L->g, kForceBlock, slab_p, slab_g);
     LQCD_DISPATCH_DS(L, k_force_store<D, S, S><<<grid_for(L->g.nsite, kForceBlock), kForceBlock, 0,
                                                 L->ctx->stream>>>((const vec2_t<S>*)U, L->g,
-                                                                  (S)md_force_scale(L->size), d_out, scale));
+                                                                  (S)md_force_scale(L->size), d_out, scale, slab_p,
+                                                                  slab_g));
     prof_end(L->ctx, &ev);
     return hipGetLastError();
 }
