@@ -659,7 +659,7 @@ int device_to_file(int fd, const char* src, uint64_t n, hipStream_t s, PinnedRin
 
 int write_bincode(lqcd_lattice* L, double beta, int with_e, uint64_t t, const char* path)
 {
-    DeviceGuard dg(L->ctx->device);
+    LATTICE_GUARD(L);
     hipStream_t s = L->ctx->stream;
     const uint64_t ne = with_e ? (uint64_t)L->nlink * 64 : 0, nl = (uint64_t)L->nlink * 144;
     DevBuf stage;
@@ -705,7 +705,7 @@ int read_bincode_into(lqcd_lattice* L, const char* path, int with_e, double* bet
             return fail(LQCD_ERR_INCOMPATIBLE_SIZE, "the state's lattice does not match the handle's extents");
     if (b.size != L->size)
         return fail(LQCD_ERR_INCOMPATIBLE_SIZE, "the state's lattice spacing does not match the handle's");
-    DeviceGuard dg(L->ctx->device);
+    LATTICE_GUARD(L);
     hipStream_t s = L->ctx->stream;
     const uint64_t ne = with_e ? (uint64_t)L->nlink * 64 : 0, nl = (uint64_t)L->nlink * 144;
     DevBuf stage;

@@ -41,6 +41,12 @@ struct DevBuf {
                                 std::string(#expr) + ": " + hipGetErrorString(_e));    \
     } while (0)
 
+// device of lattice L, with its links in site order: for entry points whose
+// kernels read or write the links by site
+#define LATTICE_GUARD(L)                                                               \
+    DeviceGuard dg((L)->ctx->device);                                                  \
+    HIP_TRY(::lqcd::site_order_links(L))
+
 #define CHECK_ARG(cond, msg)                                                           \
     do {                                                                               \
         if (!(cond)) return ::lqcd::fail(LQCD_ERR_INVALID_ARGUMENT, msg);              \

@@ -33,6 +33,26 @@
         }                                                                           \
     } while (0)
 
+// as LQCD_DISPATCH_DS, with PO: the lattice's links are in parity order (f64
+// storage only)
+#define LQCD_DISPATCH_DS_PO(L, ...)                                                 \
+    do {                                                                            \
+        if ((L)->parity_order) {                                                    \
+            constexpr bool PO = true;                                               \
+            using S = double;                                                       \
+            if ((L)->precision != 0) return hipErrorInvalidValue;                   \
+            switch ((L)->g.dim) {                                                   \
+            case 2: { constexpr int D = 2; __VA_ARGS__; } break;                    \
+            case 3: { constexpr int D = 3; __VA_ARGS__; } break;                    \
+            case 4: { constexpr int D = 4; __VA_ARGS__; } break;                    \
+            default: return hipErrorInvalidValue;                                   \
+            }                                                                       \
+        } else {                                                                    \
+            constexpr bool PO = false;                                              \
+            LQCD_DISPATCH_DS(L, __VA_ARGS__);                                       \
+        }                                                                           \
+    } while (0)
+
 namespace lqcd {
 inline unsigned grid_for(int64_t n, int block = kBlock)
 {

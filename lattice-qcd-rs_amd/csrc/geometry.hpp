@@ -80,6 +80,34 @@ inline void slab_shape(const Geom& g, int64_t block, int64_t& P, int64_t& G)
 }
 
 template <int D>
+__device__ __forceinline__ int site_parity(const Geom& g, int64_t s);
+
+// Index of a site in a link plane, from its site index and its number of steps
+// from site s.  Site order: the site index.  Parity order (PO, lattices of
+// even extents): the sites of even parity first, then the odd ones, each in
+// site order; of sites 2k and 2k + 1 one has either parity, so site s is word
+// s / 2 of its half.
+template <int D, bool PO>
+struct SiteMap {
+    int64_t off[2] = {0, 0};   // first word of the half of s, and of the other
+
+    __device__ __forceinline__ SiteMap(const Geom& g, int64_t s) : SiteMap(g, PO ? site_parity<D>(g, s) : 0) {}
+    __device__ __forceinline__ SiteMap(const Geom& g, int parity)
+    {
+        if constexpr (PO) {
+            off[0] = parity ? g.nsite / 2 : 0;
+            off[1] = g.nsite / 2 - off[0];
+        }
+    }
+    template <int STEPS>
+    __device__ __forceinline__ int64_t at(int64_t s) const
+    {
+        if constexpr (PO) return (s >> 1) + off[STEPS & 1];
+        return s;
+    }
+};
+
+template <int D>
 __device__ __forceinline__ int site_parity(const Geom& g, int64_t s)
 {
     uint32_t r = (uint32_t)s;

@@ -36,6 +36,10 @@ struct lqcd_lattice {
     size_t elem = 8;         // bytes of one stored real
     void* U[3] = {nullptr, nullptr, nullptr};
     int cur = 0;             // buffer holding the current links
+    // the current links are in parity order (SiteMap in geometry.hpp): set by
+    // the f64 checkerboard sweeps, undone by site_order_links before anything
+    // that reads them in site order
+    bool parity_order = false;
     void* E = nullptr;
     double* partials = nullptr;  // per-block reduction scratch
     double* result = nullptr;    // device reduction results
@@ -120,6 +124,7 @@ constexpr int kStreamReadBlocks = 8192;
 hipError_t launch_stream_read(hipStream_t stream, const void* src, size_t bytes, uint32_t* sink);
 
 // ---- observables (k_observables.hip) ----
+// launch_plaquette_sum and launch_force_store read links in either order
 // out[0..1] = sum Tr P (complex), out[2] = sum (1 - Re Tr P / 3)
 hipError_t launch_plaquette_sum(const lqcd_lattice* L, const void* U, double* d_out3);
 // the plaquette sums (d_out4[0..2], as launch_plaquette_sum) and the E energy
@@ -180,6 +185,10 @@ hipError_t launch_metropolis_class(const lqcd_lattice* L, void* U, int mu, int p
 hipError_t launch_metropolis_class_rng(const lqcd_lattice* L, void* U, int mu, int parity, double beta,
                                        size_t n_update, double spread, uint64_t seed, uint64_t counter);
 
+// links of buffer `in` in site order to parity order in buffer `out`, or back
+hipError_t launch_reorder_links(const lqcd_lattice* L, const void* in, void* out, bool to_parity);
+// the lattice's current links back in site order (enqueued; capi.cpp)
+hipError_t site_order_links(lqcd_lattice* L);
 // heat bath / overrelaxation of one (mu, parity) class (k_mc.hip); the heat
 // bath writes the per-link count of exhausted samplers to mh_acc (mh_p = 0)
 hipError_t launch_heat_bath_class(const lqcd_lattice* L, void* U, int mu, int parity, double beta, uint64_t seed,

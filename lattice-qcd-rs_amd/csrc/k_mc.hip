@@ -87,9 +87,10 @@ __device__ __forceinline__ uint64_t device_accept_word(uint64_t l, uint64_t seed
 // staple A_mu(x) of monte_carlo/mod.rs:339-362 in double arithmetic:
 // sum_{nu != mu} U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+ + U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
 // R12: links read as two rows (load_link_r12), for links in SU(3)
-template <int D, typename S, bool R12 = false>
+// PO: links in parity order, sm the map of site s
+template <int D, typename S, bool R12 = false, bool PO = false>
 __device__ __forceinline__ void mc_staple(const vec2_t<S>* __restrict__ U, const Geom& g, int mu, int64_t s,
-                                          mat3<double>& a)
+                                          const SiteMap<D, PO>& sm, mat3<double>& a)
 {
     const Neighbours<D> nb = neighbours<D>(g, s);
     set_zero(a);
@@ -98,20 +99,20 @@ __device__ __forceinline__ void mc_staple(const vec2_t<S>* __restrict__ U, const
     for (int nu = 0; nu < D; ++nu) {
         if (nu == mu) continue;
         {
-            const mat3<double> x = load_link_sel<R12, double, S>(U, g.npad, nu, s_pmu);
-            const mat3<double> y = load_link_sel<R12, double, S>(U, g.npad, mu, s + nb.up[nu]);
+            const mat3<double> x = load_link_sel<R12, double, S>(U, g.npad, nu, sm.template at<1>(s_pmu));
+            const mat3<double> y = load_link_sel<R12, double, S>(U, g.npad, mu, sm.template at<1>(s + nb.up[nu]));
             mat3<double> xy;
             mul<false, true>(x, y, xy);
-            const mat3<double> z = load_link_sel<R12, double, S>(U, g.npad, nu, s);
+            const mat3<double> z = load_link_sel<R12, double, S>(U, g.npad, nu, sm.template at<0>(s));
             mul_add<false, true>(xy, z, a);
         }
         {
             const int64_t s_mnu = s + nb.dn[nu];
-            const mat3<double> x = load_link_sel<R12, double, S>(U, g.npad, nu, s_pmu + nb.dn[nu]);
-            const mat3<double> y = load_link_sel<R12, double, S>(U, g.npad, mu, s_mnu);
+            const mat3<double> x = load_link_sel<R12, double, S>(U, g.npad, nu, sm.template at<2>(s_pmu + nb.dn[nu]));
+            const mat3<double> y = load_link_sel<R12, double, S>(U, g.npad, mu, sm.template at<1>(s_mnu));
             mat3<double> xy;
             mul<true, true>(x, y, xy);
-            const mat3<double> z = load_link_sel<R12, double, S>(U, g.npad, nu, s_mnu);
+            const mat3<double> z = load_link_sel<R12, double, S>(U, g.npad, nu, sm.template at<1>(s_mnu));
             mul_add<false, false>(xy, z, a);
         }
     }
@@ -126,6 +127,9 @@ __device__ __forceinline__ int64_t class_site(const Geom& g, int64_t k, int pari
     return s0 + ((site_parity<D>(g, s0) + parity) & 1);
 }
 
+// Links of f64 lattices past the L2 are in parity order here (SiteMap, PO;
+// class_order_links in capi.cpp), others in site order.
+//
 // Order of a class launch's workgroups: each covers 2 kBlock consecutive
 // sites (kBlock class links); XCD k gets a contiguous range of them
 // (xcd_remap), walked slab by slab of the slowest direction with that
@@ -145,7 +149,7 @@ __device__ __forceinline__ int64_t class_index(const ClassOrder& co)
     return logical * kBlock + threadIdx.x;
 }
 
-template <int D, typename S, bool RNG, bool R12 = false>
+template <int D, typename S, bool RNG, bool R12, bool PO>
 __global__ __launch_bounds__(kBlock) void k_metropolis(vec2_t<S>* __restrict__ U, Geom g, int mu,
                                                        int parity, double beta, int n_update,
                                                        const double* __restrict__ proposals,
@@ -159,8 +163,10 @@ __global__ __launch_bounds__(kBlock) void k_metropolis(vec2_t<S>* __restrict__ U
     if (k >= half) return;
     const int64_t s = class_site<D>(g, k, parity);
     mat3<double> a;
-    mc_staple<D, S, R12>(U, g, mu, s, a);
-    const mat3<double> u = load_link_sel<R12, double, S>(U, g.npad, mu, s);
+    const SiteMap<D, PO> sm(g, parity);
+    const int64_t own = sm.template at<0>(s);
+    mc_staple<D, S, R12, PO>(U, g, mu, s, sm, a);
+    const mat3<double> u = load_link_sel<R12, double, S>(U, g.npad, mu, own);
     const int64_t li = s * D + mu;
     const int64_t nlink = g.nsite * D;
     mat3<double> nw = u;
@@ -197,7 +203,7 @@ __global__ __launch_bounds__(kBlock) void k_metropolis(vec2_t<S>* __restrict__ U
     const int64_t o = (int64_t)(mu * 2 + parity) * half + k;
     p_out[o] = p;
     acc_out[o] = accept ? 1u : 0u;
-    if (accept) store_link<double, S>(U, g.npad, mu, s, nw);
+    if (accept) store_link<double, S>(U, g.npad, mu, own, nw);
 }
 
 // MetropolisHastingsDeltaDiagnostic::next_element_default
@@ -219,7 +225,7 @@ __global__ __launch_bounds__(64) void k_metropolis_link(vec2_t<S>* __restrict__ 
     const int64_t s = (int64_t)__umul64hi(w, (uint64_t)g.nsite);
     const int mu = (int)(((uint64_t)o.z * (uint64_t)D) >> 32);
     mat3<double> a, r, nw;
-    mc_staple<D, S>(U, g, mu, s, a);
+    mc_staple<D, S>(U, g, mu, s, SiteMap<D, false>(g, 0), a);
     const mat3<double> u = load_link<double, S>(U, g.npad, mu, s);
     const int64_t li = s * D + mu;
     device_proposal((uint64_t)li, 0, seed, counter, spread, r);
@@ -343,7 +349,7 @@ __device__ __forceinline__ void sub_block_rc(int grp, int& i, int& j)
     j = grp == 0 ? 1 : 2;
 }
 
-template <int D, typename S>
+template <int D, typename S, bool PO>
 __global__ __launch_bounds__(kBlock) void k_heat_bath(vec2_t<S>* __restrict__ U, Geom g, int mu, int parity,
                                                       double beta, uint64_t seed, uint64_t counter,
                                                       double* __restrict__ p_out, uint32_t* __restrict__ exhausted,
@@ -353,8 +359,10 @@ __global__ __launch_bounds__(kBlock) void k_heat_bath(vec2_t<S>* __restrict__ U,
     if (k >= g.nsite / 2) return;
     const int64_t s = class_site<D>(g, k, parity);
     mat3<double> a;
-    mc_staple<D, S>(U, g, mu, s, a);
-    const mat3<double> u = load_link<double, S>(U, g.npad, mu, s);
+    const SiteMap<D, PO> sm(g, parity);
+    const int64_t own = sm.template at<0>(s);
+    mc_staple<D, S, false, PO>(U, g, mu, s, sm, a);
+    const mat3<double> u = load_link<double, S>(U, g.npad, mu, own);
     const int64_t li = s * D + mu;
     mat3<double> ua, acc;
     mul<false, false>(u, a, ua);
@@ -386,7 +394,7 @@ __global__ __launch_bounds__(kBlock) void k_heat_bath(vec2_t<S>* __restrict__ U,
     }
     mat3<double> nw;
     mul<false, false>(acc, u, nw);
-    store_link<double, S>(U, g.npad, mu, s, nw);
+    store_link<double, S>(U, g.npad, mu, own, nw);
     const int64_t o = (int64_t)(mu * 2 + parity) * (g.nsite / 2) + k;
     p_out[o] = 0.0;
     exhausted[o] = ex;
@@ -514,7 +522,7 @@ __device__ __forceinline__ void svd3_jacobi(const mat3<double>& a, mat3<double>&
 //   staple^+ = W S V^+, new link = W reverse(W^+ U V) V^+, where su3::reverse
 //   (su3.rs:705-714) negates the off-diagonal entries.  The result does not
 //   depend on the phases or the order of the singular vectors.
-template <int D, typename S, bool REVERSE>
+template <int D, typename S, bool REVERSE, bool PO>
 __global__ __launch_bounds__(kBlock) void k_overrelax(vec2_t<S>* __restrict__ U, Geom g, int mu, int parity,
                                                       ClassOrder co)
 {
@@ -522,12 +530,14 @@ __global__ __launch_bounds__(kBlock) void k_overrelax(vec2_t<S>* __restrict__ U,
     if (k >= g.nsite / 2) return;
     const int64_t s = class_site<D>(g, k, parity);
     mat3<double> a, ad, t, nw;
-    mc_staple<D, S>(U, g, mu, s, a);
+    const SiteMap<D, PO> sm(g, parity);
+    const int64_t own = sm.template at<0>(s);
+    mc_staple<D, S, false, PO>(U, g, mu, s, sm, a);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) ad.e[i * 3 + j] = {a.e[j * 3 + i].re, -a.e[j * 3 + i].im};
-    const mat3<double> u = load_link<double, S>(U, g.npad, mu, s);
+    const mat3<double> u = load_link<double, S>(U, g.npad, mu, own);
     if (REVERSE) {
         mat3<double> w, v, m;
         svd3_jacobi(ad, w, v);
@@ -546,7 +556,31 @@ __global__ __launch_bounds__(kBlock) void k_overrelax(vec2_t<S>* __restrict__ U,
         mul<false, true>(rot, u, t);
         mul<false, false>(t, rot, nw);
     }
-    store_link<double, S>(U, g.npad, mu, s, nw);
+    store_link<double, S>(U, g.npad, mu, own, nw);
+}
+
+// Links in site order -> parity order (TO_PARITY) or back, one link per thread
+template <int D, typename S, bool TO_PARITY>
+__global__ __launch_bounds__(kBlock) void k_reorder_links(const vec2_t<S>* __restrict__ in, vec2_t<S>* __restrict__ out,
+                                                          Geom g)
+{
+    const int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int mu = blockIdx.y;
+    if (s >= g.nsite) return;
+    const int64_t w = SiteMap<D, true>(g, s).template at<0>(s);
+    store_link<S, S>(out, g.npad, mu, TO_PARITY ? w : s, load_link<S, S>(in, g.npad, mu, TO_PARITY ? s : w));
+}
+
+hipError_t launch_reorder_links(const lqcd_lattice* L, const void* in, void* out, bool to_parity)
+{
+    const dim3 grid(grid_for(L->g.nsite), (unsigned)L->g.dim);
+    if (to_parity)
+        LQCD_DISPATCH_DS(L, k_reorder_links<D, S, true><<<grid, kBlock, 0, L->ctx->stream>>>(
+                                (const vec2_t<S>*)in, (vec2_t<S>*)out, L->g));
+    else
+        LQCD_DISPATCH_DS(L, k_reorder_links<D, S, false><<<grid, kBlock, 0, L->ctx->stream>>>(
+                                (const vec2_t<S>*)in, (vec2_t<S>*)out, L->g));
+    return hipGetLastError();
 }
 
 // the slab order of a class launch when the lattice allows it: whole
@@ -564,7 +598,7 @@ hipError_t launch_heat_bath_class(const lqcd_lattice* L, void* U, int mu, int pa
     const unsigned grid = grid_for(L->g.nsite / 2);
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_HEAT_BATH, &ev);
-    LQCD_DISPATCH_DS(L, k_heat_bath<D, S><<<grid, kBlock, 0, L->ctx->stream>>>(
+    LQCD_DISPATCH_DS_PO(L, k_heat_bath<D, S, PO><<<grid, kBlock, 0, L->ctx->stream>>>(
                             (vec2_t<S>*)U, L->g, mu, parity, beta, seed, counter, L->mh_p, L->mh_acc,
                             class_order(L)));
     prof_end(L->ctx, &ev);
@@ -577,10 +611,10 @@ hipError_t launch_overrelax_class(const lqcd_lattice* L, void* U, int mu, int pa
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_OVERRELAX, &ev);
     if (reverse)
-        LQCD_DISPATCH_DS(L, k_overrelax<D, S, true><<<grid, kBlock, 0, L->ctx->stream>>>((vec2_t<S>*)U, L->g,
+        LQCD_DISPATCH_DS_PO(L, k_overrelax<D, S, true, PO><<<grid, kBlock, 0, L->ctx->stream>>>((vec2_t<S>*)U, L->g,
                                                                                          mu, parity, class_order(L)));
     else
-        LQCD_DISPATCH_DS(L, k_overrelax<D, S, false><<<grid, kBlock, 0, L->ctx->stream>>>((vec2_t<S>*)U, L->g,
+        LQCD_DISPATCH_DS_PO(L, k_overrelax<D, S, false, PO><<<grid, kBlock, 0, L->ctx->stream>>>((vec2_t<S>*)U, L->g,
                                                                                           mu, parity, class_order(L)));
     prof_end(L->ctx, &ev);
     return hipGetLastError();
@@ -593,7 +627,7 @@ hipError_t launch_metropolis_class(const lqcd_lattice* L, void* U, int mu, int p
     const unsigned grid = grid_for(L->g.nsite / 2);
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_METROPOLIS, &ev);
-    LQCD_DISPATCH_DS(L, k_metropolis<D, S, false><<<grid, kBlock, 0, L->ctx->stream>>>(
+    LQCD_DISPATCH_DS_PO(L, k_metropolis<D, S, false, false, PO><<<grid, kBlock, 0, L->ctx->stream>>>(
                             (vec2_t<S>*)U, L->g, mu, parity, beta, (int)n_update, d_proposals,
                             d_uniforms, 0.0, 0, 0, L->mh_p, L->mh_acc, class_order(L)));
     prof_end(L->ctx, &ev);
@@ -615,11 +649,11 @@ hipError_t launch_metropolis_class_rng(const lqcd_lattice* L, void* U, int mu, i
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_METROPOLIS, &ev);
     if (L->md_r12)
-        LQCD_DISPATCH_DS(L, k_metropolis<D, S, true, true><<<grid, kBlock, 0, L->ctx->stream>>>(
+        LQCD_DISPATCH_DS_PO(L, k_metropolis<D, S, true, true, PO><<<grid, kBlock, 0, L->ctx->stream>>>(
                                 (vec2_t<S>*)U, L->g, mu, parity, beta, (int)n_update, nullptr, nullptr,
                                 spread, seed, counter, L->mh_p, L->mh_acc, class_order(L)));
     else
-        LQCD_DISPATCH_DS(L, k_metropolis<D, S, true, false><<<grid, kBlock, 0, L->ctx->stream>>>(
+        LQCD_DISPATCH_DS_PO(L, k_metropolis<D, S, true, false, PO><<<grid, kBlock, 0, L->ctx->stream>>>(
                                 (vec2_t<S>*)U, L->g, mu, parity, beta, (int)n_update, nullptr, nullptr,
                                 spread, seed, counter, L->mh_p, L->mh_acc, class_order(L)));
     prof_end(L->ctx, &ev);

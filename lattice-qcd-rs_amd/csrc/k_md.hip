@@ -52,7 +52,7 @@ namespace lqcd {
 // and 1 % (f32) larger, so all nine entries are read.
 constexpr int kForceBlock = 128;
 
-template <int D, typename S, typename T>
+template <int D, typename S, typename T, bool PO>
 __global__ __launch_bounds__(kForceBlock) void k_force_store(const vec2_t<S>* __restrict__ U, Geom g,
                                                              T fscale, double* __restrict__ out,
                                                              double oscale, int64_t slab_p, int64_t slab_g)
@@ -66,10 +66,11 @@ __global__ __launch_bounds__(kForceBlock) void k_force_store(const vec2_t<S>* __
     if (s < g.nsite) {
         const Neighbours<D> nb = neighbours<D>(g, s);
         mat3<T> sig[D];
-        staple_sums_site<D, S, T>(U, g, s, nb, sig);
+        staple_sums_site<D, S, T, false, false, PO>(U, g, s, nb, sig);
+        const int64_t own = SiteMap<D, PO>(g, s).template at<0>(s);
 #pragma unroll
         for (int mu = 0; mu < D; ++mu) {
-            const mat3<T> u = load_link<T, S>(U, g.npad, mu, s);
+            const mat3<T> u = load_link<T, S>(U, g.npad, mu, own);
             mat3<T> m;
             mul<false, false>(u, sig[mu], m);
             T f[8];
@@ -413,10 +414,9 @@ hipError_t launch_force_store(const lqcd_lattice* L, const void* U, double* d_ou
     prof_begin(L->ctx, PROF_FORCE_STORE, &ev);
     int64_t slab_p, slab_g;
     slab_shape(L->g, kForceBlock, slab_p, slab_g);
-    LQCD_DISPATCH_DS(L, k_force_store<D, S, S><<<grid_for(L->g.nsite, kForceBlock), kForceBlock, 0,
-                                                L->ctx->stream>>>((const vec2_t<S>*)U, L->g,
-                                                                  (S)md_force_scale(L->size), d_out, scale, slab_p,
-                                                                  slab_g));
+    const unsigned grid = grid_for(L->g.nsite, kForceBlock);
+    LQCD_DISPATCH_DS_PO(L, k_force_store<D, S, S, PO><<<grid, kForceBlock, 0, L->ctx->stream>>>(
+                               (const vec2_t<S>*)U, L->g, (S)md_force_scale(L->size), d_out, scale, slab_p, slab_g));
     prof_end(L->ctx, &ev);
     return hipGetLastError();
 }

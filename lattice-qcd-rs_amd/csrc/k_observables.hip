@@ -11,14 +11,14 @@
 namespace lqcd {
 
 // plaquette_site summed over the lattice
-template <int D, typename S>
+template <int D, typename S, bool PO>
 __global__ __launch_bounds__(kBlock) void k_plaquette_partials(const vec2_t<S>* __restrict__ U, Geom g,
                                                                double* __restrict__ partials)
 {
     double acc[3] = {0.0, 0.0, 0.0};
     const int64_t step = (int64_t)gridDim.x * kBlock;
     for (int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x; s < g.nsite; s += step)
-        plaquette_site<D, S>(U, g, s, acc);
+        plaquette_site<D, S, PO>(U, g, s, acc);
     block_reduce_to<3>(acc, partials + (int64_t)blockIdx.x * kReduceSlots);
 }
 
@@ -131,7 +131,7 @@ hipError_t launch_plaquette_sum(const lqcd_lattice* L, const void* U, double* d_
     const int nb = reduce_blocks(L->g.nsite);
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_PLAQUETTE, &ev);
-    LQCD_DISPATCH_DS(L, k_plaquette_partials<D, S><<<nb, kBlock, 0, L->ctx->stream>>>(
+    LQCD_DISPATCH_DS_PO(L, k_plaquette_partials<D, S, PO><<<nb, kBlock, 0, L->ctx->stream>>>(
                             (const vec2_t<S>*)U, L->g, L->partials));
     prof_end(L->ctx, &ev);
     k_final_reduce<3><<<1, kBlock, 0, L->ctx->stream>>>(L->partials, nb, d_out3);

@@ -105,13 +105,15 @@ __device__ __forceinline__ void own_put(vec2_t<T>* own, int mu, const mat3<T>& m
 // All D staple sums of site s.  Upper staples pairwise through
 // W = U_nu(x+mu) U_mu(x+nu)^+:  Sigma_mu += W U_nu(x)^+,
 // Sigma_nu += W^+ U_mu(x)^+.
-template <int D, typename S, typename T, bool R12 = false, bool OWN = false>
+// PO: links in parity order (SiteMap).
+template <int D, typename S, typename T, bool R12 = false, bool OWN = false, bool PO = false>
 __device__ __forceinline__ void staple_sums_site(const vec2_t<S>* __restrict__ U, const Geom& g,
                                                  int64_t s, const Neighbours<D>& nb,
                                                  mat3<T> (&sig)[D], const vec2_t<T>* own = nullptr)
 {
 #pragma unroll
     for (int mu = 0; mu < D; ++mu) set_zero(sig[mu]);
+    static_assert(!(R12 && PO), "two-row reads are built for site order only");
     if constexpr (R12) {
         // links, W and staples in SU(3): products as rows 0, 1 (mul_rows01);
         // W gets its row 2 rebuilt (it is used as W^+), the staples theirs
@@ -155,34 +157,35 @@ __device__ __forceinline__ void staple_sums_site(const vec2_t<S>* __restrict__ U
         }
         return;
     }
+    const SiteMap<D, PO> sm(g, s);
 #pragma unroll
     for (int mu = 0; mu < D; ++mu)
 #pragma unroll
         for (int nu = mu + 1; nu < D; ++nu) {
             mat3<T> w;
             {
-                const mat3<T> a = load_link_sel<R12, T, S>(U, g.npad, nu, s + nb.up[mu]);
-                const mat3<T> b = load_link_sel<R12, T, S>(U, g.npad, mu, s + nb.up[nu]);
+                const mat3<T> a = load_link_sel<R12, T, S>(U, g.npad, nu, sm.template at<1>(s + nb.up[mu]));
+                const mat3<T> b = load_link_sel<R12, T, S>(U, g.npad, mu, sm.template at<1>(s + nb.up[nu]));
                 mul<false, true>(a, b, w);
             }
             {
-                const mat3<T> c = load_link_sel<R12, T, S>(U, g.npad, nu, s);
+                const mat3<T> c = load_link_sel<R12, T, S>(U, g.npad, nu, sm.template at<0>(s));
                 mul_add<false, true>(w, c, sig[mu]);
             }
             {
-                const mat3<T> c = load_link_sel<R12, T, S>(U, g.npad, mu, s);
+                const mat3<T> c = load_link_sel<R12, T, S>(U, g.npad, mu, sm.template at<0>(s));
                 mul_add<true, true>(w, c, sig[nu]);
             }
         }
 #pragma unroll
     for (int nu = 0; nu < D; ++nu) {
         const int64_t s_mnu = s + nb.dn[nu];
-        const mat3<T> c = load_link_sel<R12, T, S>(U, g.npad, nu, s_mnu);
+        const mat3<T> c = load_link_sel<R12, T, S>(U, g.npad, nu, sm.template at<1>(s_mnu));
 #pragma unroll
         for (int mu = 0; mu < D; ++mu) {
             if (mu == nu) continue;
-            const mat3<T> a = load_link_sel<R12, T, S>(U, g.npad, nu, s_mnu + nb.up[mu]);
-            const mat3<T> b = load_link_sel<R12, T, S>(U, g.npad, mu, s_mnu);
+            const mat3<T> a = load_link_sel<R12, T, S>(U, g.npad, nu, sm.template at<2>(s_mnu + nb.up[mu]));
+            const mat3<T> b = load_link_sel<R12, T, S>(U, g.npad, mu, sm.template at<1>(s_mnu));
             mat3<T> ab;
             mul<true, true>(a, b, ab);
             mul_add<false, false>(ab, c, sig[mu]);

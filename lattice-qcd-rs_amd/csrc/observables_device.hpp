@@ -11,19 +11,21 @@ namespace lqcd {
 // to acc[0..2], with P_ij(x) = U_i(x) U_j(x+i) U_i(x+j)^+ U_j(x)^+
 // (LinkMatrix::pij, src/field.rs:761-771) taken as
 // Tr[(U_i(x) U_j(x+i)) (U_j(x) U_i(x+j))^+], in double arithmetic.
-template <int D, typename S>
+// PO: links in parity order (SiteMap).
+template <int D, typename S, bool PO = false>
 __device__ __forceinline__ void plaquette_site(const vec2_t<S>* __restrict__ U, const Geom& g, int64_t s,
                                                double* acc)
 {
     const Neighbours<D> nb = neighbours<D>(g, s);
+    const SiteMap<D, PO> sm(g, s);
 #pragma unroll
     for (int i = 0; i < D; ++i) {
 #pragma unroll
         for (int j = i + 1; j < D; ++j) {
-            const mat3<double> ui = load_link<double, S>(U, g.npad, i, s);
-            const mat3<double> uj = load_link<double, S>(U, g.npad, j, s);
-            const mat3<double> uj_pi = load_link<double, S>(U, g.npad, j, s + nb.up[i]);
-            const mat3<double> ui_pj = load_link<double, S>(U, g.npad, i, s + nb.up[j]);
+            const mat3<double> ui = load_link<double, S>(U, g.npad, i, sm.template at<0>(s));
+            const mat3<double> uj = load_link<double, S>(U, g.npad, j, sm.template at<0>(s));
+            const mat3<double> uj_pi = load_link<double, S>(U, g.npad, j, sm.template at<1>(s + nb.up[i]));
+            const mat3<double> ui_pj = load_link<double, S>(U, g.npad, i, sm.template at<1>(s + nb.up[j]));
             mat3<double> a, b;
             mul<false, false>(ui, uj_pi, a);
             mul<false, false>(uj, ui_pj, b);
