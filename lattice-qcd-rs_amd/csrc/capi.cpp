@@ -528,6 +528,8 @@ int lqcd_lattice_destroy(lqcd_lattice* L)
     if (L->md_partials) (void)hipFree(L->md_partials);
     for (int k = 0; k < 3; ++k)
         if (L->gauss_e[k]) (void)hipFree(L->gauss_e[k]);
+    for (int k = 0; k < 2; ++k)
+        if (L->gauss_t[k]) (void)hipFree(L->gauss_t[k]);
     for (auto& ge : L->md_graph)
         if (ge) (void)hipGraphExecDestroy(ge);
     delete L;
@@ -745,14 +747,22 @@ int lqcd_efield_project_gauss(lqcd_lattice* L, size_t max_iter, size_t* iteratio
     if (int rc = ensure_gauss_buffers(L)) return rc;
     // project_to_gauss, src/field.rs:1265-1294: one step, then while the
     // deviation is above N * 4 * 8 * 10 * eps, four more steps.  Each step is
-    // one k_gauss_fused launch, which also sums the deviation of its input: a
-    // check is the first launch of its group of four.  The host reads that
+    // one launch, which also sums the deviation of its input: a
+    // check is the first launch of its group of four, the only one whose sum is
+    // reduced.  The host reads that
     // deviation while the other three steps run; they write the two buffers
     // other than the checked field, which stays the result if the check passes.
     double* const buf[3] = {L->gauss_e[0], L->gauss_e[1], L->gauss_e[2]};
+    double* tr[2] = {nullptr, nullptr};   // transports; tr[1] goes with buf[cur] at a check
+    if (gauss_uses_transports(L))
+        for (int k = 0; k < 2; ++k) {
+            if (!L->gauss_t[k])
+                HIP_TRY(hipMalloc((void**)&L->gauss_t[k], sizeof(double) * 9 * (size_t)L->g.npad * L->g.dim));
+            tr[k] = L->gauss_t[k];
+        }
     int cur = 1;
-    HIP_TRY(launch_efield_to_double(L, L->E, buf[0]));
-    HIP_TRY(launch_gauss_fused(L, buf[0], buf[1], L->result + 1));
+    HIP_TRY(launch_gauss_start(L, buf[0], tr[0]));
+    HIP_TRY(launch_gauss_step(L, buf[0], tr[0], buf[1], tr[1], nullptr));
     const double threshold = 2.220446049250313e-16 * (double)(L->g.nsite * 4 * 8 * 10);
     hipEvent_t checked;
     HIP_TRY(hipEventCreateWithFlags(&checked, hipEventDisableTiming));
@@ -765,12 +775,12 @@ int lqcd_efield_project_gauss(lqcd_lattice* L, size_t max_iter, size_t* iteratio
     double div = 0.0;
     for (; it < max_iter; ++it) {
         const int n1 = (cur + 1) % 3, n2 = (cur + 2) % 3;
-        HIP_TRY(launch_gauss_fused(L, buf[cur], buf[n1], L->result));
+        HIP_TRY(launch_gauss_step(L, buf[cur], tr[1], buf[n1], tr[0], L->result));
         HIP_TRY(hipMemcpyAsync(L->host_result, L->result, sizeof(double), hipMemcpyDeviceToHost, L->ctx->stream));
         HIP_TRY(hipEventRecord(checked, L->ctx->stream));
-        HIP_TRY(launch_gauss_fused(L, buf[n1], buf[n2], L->result + 1));
-        HIP_TRY(launch_gauss_fused(L, buf[n2], buf[n1], L->result + 1));
-        HIP_TRY(launch_gauss_fused(L, buf[n1], buf[n2], L->result + 1));
+        HIP_TRY(launch_gauss_step(L, buf[n1], tr[0], buf[n2], tr[1], nullptr));
+        HIP_TRY(launch_gauss_step(L, buf[n2], tr[1], buf[n1], tr[0], nullptr));
+        HIP_TRY(launch_gauss_step(L, buf[n1], tr[0], buf[n2], tr[1], nullptr));
         HIP_TRY(hipEventSynchronize(checked));
         div = L->host_result[0];
         if (std::isnan(div)) {

@@ -68,6 +68,55 @@ __device__ __forceinline__ int64_t slab_block(int64_t j, int64_t P, int64_t G)
     return (q * G + r % G) * P + r / G;
 }
 
+// Coordinates of site s, and the offsets to its neighbours along a direction
+// that is known at run time only (uniform over the wave: the extents come
+// through scalar registers and the coordinate through a few selects, where an
+// indexed Neighbours would go through LDS).
+template <int D>
+struct SiteCoords {
+    uint32_t x[D];
+
+    __device__ __forceinline__ SiteCoords(const Geom& g, int64_t s)
+    {
+        uint32_t r = (uint32_t)s;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const uint32_t L = (uint32_t)g.extent[d];
+            x[d] = (d == D - 1) ? r : r % L;
+            r /= L;
+        }
+    }
+    __device__ __forceinline__ uint32_t at(int d) const
+    {
+        uint32_t v = x[0];
+#pragma unroll
+        for (int k = 1; k < D; ++k) v = d == k ? x[k] : v;
+        return v;
+    }
+    __device__ __forceinline__ void extent(const Geom& g, int d, int32_t& L, int32_t& st) const
+    {
+        L = g.extent[0];
+        st = 1;
+#pragma unroll
+        for (int k = 1; k < D; ++k) {
+            L = d == k ? g.extent[k] : L;
+            st = d == k ? (int32_t)g.stride[k] : st;
+        }
+    }
+    __device__ __forceinline__ int32_t up(const Geom& g, int d) const
+    {
+        int32_t L, st;
+        extent(g, d, L, st);
+        return (int32_t)at(d) == L - 1 ? -(L - 1) * st : st;
+    }
+    __device__ __forceinline__ int32_t dn(const Geom& g, int d) const
+    {
+        int32_t L, st;
+        extent(g, d, L, st);
+        return at(d) == 0 ? (L - 1) * st : -st;
+    }
+};
+
 // P and G of slab_block for workgroups of `block` sites, or 0 where the
 // lattice does not allow the order (whole workgroups per slice of the slowest
 // direction, 8 | its extent).

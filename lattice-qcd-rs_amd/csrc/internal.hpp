@@ -65,6 +65,7 @@ struct lqcd_lattice {
     int64_t su3_known = -1;
     void* gauss_g = nullptr;       // Gauss law G(x): 9 planes of double2
     double* gauss_e[3] = {nullptr, nullptr, nullptr};  // double copies of E for the projection
+    double* gauss_t[2] = {nullptr, nullptr};           // its transports U^+ E U
     double* md_partials = nullptr;  // the HMC's fused H sums: two sets of per-workgroup partials
 };
 
@@ -211,9 +212,16 @@ hipError_t launch_plaquette_field(const lqcd_lattice* L, int which, int a, bool 
 // G(x) of the double E copy Ed, and div = sum_x |Tr(sum_a T^a G(x))| into d_div
 hipError_t launch_gauss(const lqcd_lattice* L, const double* Ed, double* d_div);
 hipError_t launch_gauss_to_aos(const lqcd_lattice* L, double* d_out);
-// one project_to_gauss_step Ed_in -> Ed_out with G computed in the kernel
-// (gauss_g untouched), and div of Ed_in into d_div
-hipError_t launch_gauss_fused(const lqcd_lattice* L, const double* Ed_in, double* Ed_out, double* d_div);
+// whether the projection's steps carry the transports U^+ E U of E along
+bool gauss_uses_transports(const lqcd_lattice* L);
+// E to its double copy Ed, and its transports to T (9 npad doubles per
+// direction; null: steps without them)
+hipError_t launch_gauss_start(const lqcd_lattice* L, double* Ed, double* T);
+// one project_to_gauss_step (E_in, T_in) -> (E_out, T_out) with G computed in
+// the kernel (gauss_g untouched), and div of E_in into d_div (null: not
+// wanted, its reduction is left out)
+hipError_t launch_gauss_step(const lqcd_lattice* L, const double* E_in, const double* T_in, double* E_out,
+                             double* T_out, double* d_div);
 hipError_t launch_efield_to_double(const lqcd_lattice* L, const void* E, double* Ed);
 hipError_t launch_efield_from_double(const lqcd_lattice* L, const double* Ed, void* E);
 // sum of nblocks partials (slot 0) into d_out1

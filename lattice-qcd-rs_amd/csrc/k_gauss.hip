@@ -375,6 +375,138 @@ __global__ __launch_bounds__(kBlock) void k_gauss_fused(const vec2_t<S>* __restr
     block_reduce_to<1>(acc, partials + (int64_t)blockIdx.x * kReduceSlots);
 }
 
+// ---- one link per thread, transports carried along ----
+
+// The transports T_i(x) = U_i(x)^+ E_i(x) U_i(x) that the Gauss law needs are kept
+// beside E: G(x) = sum_i [E_i(x) - T_i(x - i)] is then sums of loads, and the
+// thread that steps E_i(x) has U_i(x) at hand for the next step's T_i(x).  A
+// T is Hermitian, not traceless where the links are off SU(3): nine doubles,
+// per direction four planes of 16-byte words (d0 d1 | d2 Re o0 | Im o0 Re o1 |
+// Im o1 Re o2) and one of 8-byte words (Im o2).
+__device__ __forceinline__ herm3 load_transport(const double* __restrict__ T, int64_t npad, int mu, int64_t s)
+{
+    const __amdgpu_buffer_rsrc_t r = planes_rsrc(T + (int64_t)mu * 9 * npad, npad, 9);
+    const uint32_t off = (uint32_t)s * 16u, plane = (uint32_t)npad * 16u;
+    const double2 a = buf_load<double2>(r, off, 0), b = buf_load<double2>(r, off, plane);
+    const double2 c = buf_load<double2>(r, off, 2 * plane), d = buf_load<double2>(r, off, 3 * plane);
+    herm3 h;
+    h.d[0] = a.x;
+    h.d[1] = a.y;
+    h.d[2] = b.x;
+    h.o[0] = {b.y, c.x};
+    h.o[1] = {c.y, d.x};
+    h.o[2] = {d.y, buf_load<double>(r, (uint32_t)s * 8u, 4 * plane)};
+    return h;
+}
+
+__device__ __forceinline__ void store_transport(double* __restrict__ T, int64_t npad, int mu, int64_t s, const herm3& h)
+{
+    const __amdgpu_buffer_rsrc_t r = planes_rsrc(T + (int64_t)mu * 9 * npad, npad, 9);
+    const uint32_t off = (uint32_t)s * 16u, plane = (uint32_t)npad * 16u;
+    buf_store<double2>(r, off, 0, make_double2(h.d[0], h.d[1]));
+    buf_store<double2>(r, off, plane, make_double2(h.d[2], h.o[0].re));
+    buf_store<double2>(r, off, 2 * plane, make_double2(h.o[0].im, h.o[1].re));
+    buf_store<double2>(r, off, 3 * plane, make_double2(h.o[1].im, h.o[2].re));
+    buf_store<double>(r, (uint32_t)s * 8u, 4 * plane, h.o[2].im);
+}
+
+// U^+ E U of a link
+__device__ __forceinline__ herm3 transport(const mat3<double>& u, const herm3& e)
+{
+    mat3<double> t;
+    mul_gen_herm<true>(u, e, t);
+    return mul_to_herm<false>(t, u);
+}
+
+__device__ __forceinline__ void herm_sub_add(herm3& G, const herm3& e, const herm3& t)
+{
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        G.d[j] += e.d[j] - t.d[j];
+        G.o[j] = {G.o[j].re + (e.o[j].re - t.o[j].re), G.o[j].im + (e.o[j].im - t.o[j].im)};
+    }
+}
+
+// E of the storage type into its double copy, and the transports
+template <int D, typename S>
+__global__ __launch_bounds__(kBlock) void k_gauss_start(const vec2_t<S>* __restrict__ U, const S* __restrict__ E, Geom g,
+                                                        double* __restrict__ Ed, double* __restrict__ T)
+{
+    const int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int mu = blockIdx.y;
+    if (s >= g.nsite) return;
+    double e[8];
+    load_e<double, S>(E, g.npad, mu, s, e);
+    store_e<double, double>(Ed, g.npad, mu, s, e);
+    store_transport(T, g.npad, mu, s, transport(load_link<double, S>(U, g.npad, mu, s), herm_from_adjoint(e)));
+}
+
+// One project_to_gauss_step of the whole field, E_in, T_in -> E_out, T_out,
+// and the block partials of div(E_in).  Bound by latency on the lattices that
+// take it (gauss_uses_transports): no G is evaluated by products, and all
+// loads of a link are issued before the barrier (16^4 f64 28.7 -> 27.7 us, 8^4
+// 10.4 -> 8.5).  A workgroup takes `chunk` consecutive
+// tiles of 64 sites, one link of a site per thread (wave i: direction i): the
+// waves' terms of G(x) meet in LDS, each wave forms G(x + i) itself.
+template <int D, typename S>
+__global__ __launch_bounds__(64 * D) void k_gauss_links(const vec2_t<S>* __restrict__ U, const double* __restrict__ E_in,
+                                                        const double* __restrict__ T_in, Geom g,
+                                                        double* __restrict__ E_out, double* __restrict__ T_out,
+                                                        double* __restrict__ partials, int chunk)
+{
+    __shared__ double gl[D][9 * 64];
+    const int i = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const int64_t b = xcd_remap(blockIdx.x, gridDim.x);
+    double acc[1] = {0.0};
+#pragma unroll 1
+    for (int k = 0; k < chunk; ++k) {
+        const int64_t s = (b * chunk + k) * 64 + lane;
+        const bool live = s < g.nsite;
+        const SiteCoords<D> x(g, live ? s : 0);
+        double e[8];
+        herm3 G = {}, Gn = {};
+        mat3<double> u;
+        if (live) {
+            // every load of the link before the barrier: one round of latency
+            load_e<double, double>(E_in, g.npad, i, s, e);
+            const herm3 tm = load_transport(T_in, g.npad, i, s + x.dn(g, i));
+            u = load_link<double, S>(U, g.npad, i, s);
+            const int64_t sn = s + x.up(g, i);
+#pragma unroll
+            for (int j = 0; j < D; ++j) {
+                double en[8];
+                load_e<double, double>(E_in, g.npad, j, sn, en);
+                herm_sub_add(Gn, herm_from_adjoint(en), load_transport(T_in, g.npad, j, j == i ? s : sn + x.dn(g, j)));
+            }
+            herm_sub_add(G, herm_from_adjoint(e), tm);
+            herm_put(gl[i], 64, lane, G);
+        }
+        __syncthreads();
+        if (live) {
+            G = herm_get(gl[0], 64, lane);
+#pragma unroll
+            for (int j = 1; j < D; ++j) {
+                const herm3 h = herm_get(gl[j], 64, lane);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    G.d[q] += h.d[q];
+                    G.o[q] = {G.o[q].re + h.o[q].re, G.o[q].im + h.o[q].im};
+                }
+            }
+            if (i == 0) acc[0] += gsum_trace_abs(herm_full(G));
+            gauss_step_link(u, G, Gn, e);
+            store_e<double, double>(E_out, g.npad, i, s, e);
+            store_transport(T_out, g.npad, i, s, transport(u, herm_from_adjoint(e)));
+        }
+        __syncthreads();
+    }
+    if (i == 0) {
+        wave_sum<1>(acc);
+        if (lane == 0) partials[(int64_t)blockIdx.x * kReduceSlots] = acc[0];
+    }
+}
+
 // ---- streamed tiles (D = 4) ----
 // A workgroup owns a tile of L0 x a x b sites (x_0 fastest, kBlock = L0 a b
 // threads, one site each; a wavefront holds whole x_0 rows of one x_2 layer)
@@ -625,9 +757,10 @@ static int gauss_blocks(int64_t n)
 // (or LQCD_GAUSS_TILES=0 pins the site walk): L0 divides 64 (whole x_0 rows
 // per wavefront), a tile L0 x a x b of kBlock sites with the rows of a
 // wavefront in one x_2 layer, a | L1, b | L2 and the smallest halo L0 (a + b);
-// C | L3 the largest of 32, 16, .., 1 that leaves min(512, half the tiles of the
+// C | L3 the largest of 32, 16, .., 1 that leaves min(512, the tiles of the
 // lattice) workgroups or more (512: one round of two workgroups per CU) and at
-// most kMaxReduceBlocks.
+// most kMaxReduceBlocks.  (With half the tiles as the floor the 256 tiles of 16^4
+// ran as 128 workgroups of C = 2, half the CUs: 34.4 against 29.3 us per f64 step.)
 static GaussTiles gauss_tiles(const Geom& g)
 {
     GaussTiles gt;
@@ -651,7 +784,7 @@ static GaussTiles gauss_tiles(const Geom& g)
     if (best_a == 0) return gt;
     const int64_t tiles = (int64_t)(L1 / best_a) * (L2 / best_b);
     const int64_t all = tiles * L3;
-    const int64_t target = all / 2 < 512 ? all / 2 : 512;
+    const int64_t target = all < 512 ? all : 512;
     int C = 0;
     for (int c : {32, 16, 8, 4, 2, 1})
         if (L3 % c == 0 && all / c >= target && all / c <= kMaxReduceBlocks) {
@@ -686,22 +819,54 @@ hipError_t launch_gauss(const lqcd_lattice* L, const double* Ed, double* d_div)
     return launch_final_reduce1(L, nb, d_div);
 }
 
-hipError_t launch_gauss_fused(const lqcd_lattice* L, const double* Ed_in, double* Ed_out, double* d_div)
+bool gauss_uses_transports(const lqcd_lattice* L)
 {
-    const GaussTiles gt = gauss_tiles(L->g);
+    // Small lattices, where the step is one round of memory latency and not the
+    // 1.1 - 1.7 KB per site that it moves: below 2^15 sites against the streamed
+    // tiles (f64, us per step: 16^2 x 8^2 19.0 -> 10.0, 8^4 16.4 -> 8.5;
+    // 16^3 x 8 f64 23.4 -> 16.3, but 16^4 f32 23.2 -> 25.4, 32^4 362 -> 502), and
+    // below 2^20 against the site walk, which evaluates up to D + 1 Gs per site
+    // one after the other (13x11x17x9 25.6 -> 13.5, 20x18x16x14 54.6 -> 33.2,
+    // 24^4 200 -> 167, 500^2 52.1 -> 36.3; 48^4 f32 2210 -> 2770).  Not in D = 3,
+    // where the site walk is level or ahead (8^3 7.9 / 7.9, 32^3 16.5 / 23.8, 48^3
+    // 35.5 / 38.5).
+    if (L->g.dim == 3) return false;
+    return L->g.nsite < (gauss_tiles(L->g).a > 0 ? 1 << 15 : 1 << 20);
+}
+
+hipError_t launch_gauss_start(const lqcd_lattice* L, double* Ed, double* T)
+{
+    if (!T) return launch_efield_to_double(L, L->E, Ed);
+    const dim3 grid(grid_for(L->g.nsite), (unsigned)L->g.dim);
+    LQCD_DISPATCH_DS(L, k_gauss_start<D, S><<<grid, kBlock, 0, L->ctx->stream>>>(
+                            (const vec2_t<S>*)L->U[L->cur], (const S*)L->E, L->g, Ed, T));
+    return hipGetLastError();
+}
+
+hipError_t launch_gauss_step(const lqcd_lattice* L, const double* E_in, const double* T_in, double* E_out,
+                             double* T_out, double* d_div)
+{
+    const auto* U = (const void*)L->U[L->cur];
+    hipStream_t st = L->ctx->stream;
     int nb;
-    if (gt.a > 0) {
+    if (T_in) {
+        const int64_t tiles = (L->g.nsite + 63) / 64;
+        const int chunk = (int)((tiles + kMaxReduceBlocks - 1) / kMaxReduceBlocks);
+        nb = (int)((tiles + chunk - 1) / chunk);
+        LQCD_DISPATCH_DS(L, k_gauss_links<D, S><<<nb, 64 * D, 0, st>>>((const vec2_t<S>*)U, E_in, T_in, L->g, E_out,
+                                                                        T_out, L->partials, chunk));
+    } else if (const GaussTiles gt = gauss_tiles(L->g); gt.a > 0) {
         nb = gt.nblocks;
         const size_t lds = sizeof(double) * 9 * (2 * kBlock + (size_t)L->g.extent[0] * (gt.a + gt.b));
-        LQCD_DISPATCH_S(L, k_gauss_stream<S><<<nb, kBlock, lds, L->ctx->stream>>>(
-                               (const vec2_t<S>*)L->U[L->cur], Ed_in, L->g, Ed_out, L->partials, gt));
+        LQCD_DISPATCH_S(L, k_gauss_stream<S><<<nb, kBlock, lds, st>>>((const vec2_t<S>*)U, E_in, L->g, E_out,
+                                                                       L->partials, gt));
     } else {
         nb = gauss_blocks(L->g.nsite);
-        LQCD_DISPATCH_DS(L, k_gauss_fused<D, S><<<nb, kBlock, 0, L->ctx->stream>>>(
-                                (const vec2_t<S>*)L->U[L->cur], Ed_in, L->g, Ed_out, L->partials));
+        LQCD_DISPATCH_DS(L, k_gauss_fused<D, S><<<nb, kBlock, 0, st>>>((const vec2_t<S>*)U, E_in, L->g, E_out,
+                                                                        L->partials));
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !d_div) return e;
     return launch_final_reduce1(L, nb, d_div);
 }
 
