@@ -256,8 +256,9 @@ static int buffer_after(const lqcd_lattice* L, size_t n)
 // store only the first two rows of the links they drift; the final kick of
 // the per-site kernels writes row 2 of the final links back (otherwise
 // k_complete_row2 does).  sums (non-null): the terms of H before and after
-// the integration go to result.  With a per-site work decomposition the
-// first launch and the final kick sum them on the way (MdExtra): result[0..3]
+// the integration go to result.  Where the work decomposition sums
+// (md_variant_has_sums: per site, and per link in f64) the first launch and
+// the final kick sum them on the way (MdExtra): result[0..3]
 // = sum Re Tr(U Sigma) and sum e^2 over all links, before, then after, and
 // *sums = true.  Otherwise the plaquette kernel runs before and after the MD
 // (launch_hamiltonian_sum into result[0..3] and result[4..7]), *sums = false.
@@ -274,12 +275,14 @@ int integrate_steps(lqcd_lattice* L, double dt, size_t n, int drift, int scheme,
     if (drift == LQCD_DRIFT_ADDITIVE) L->su3_known = -2;
     L->md_r12_last = L->md_r12;
     if (int rc = ensure_md_variant(L, drift)) return rc;
-    const bool site = md_variant_has_sums(L->md_variant);
-    const bool with_sums = sums && site && n > 0;
-    const int64_t nb = (int64_t)grid_for(L->g.nsite);
+    const bool site = md_variant_per_site(L->md_variant);
+    const bool with_sums = sums && md_variant_has_sums(L, L->md_variant) && n > 0;
+    const int64_t nb = md_sums_blocks(L, L->md_variant);
     if (with_sums) {
+        // two sets of partials, sized for the variant with the most workgroups
         if (!L->md_partials)
-            HIP_TRY(hipMalloc((void**)&L->md_partials, sizeof(double) * 2 * (size_t)nb * kReduceSlots));
+            HIP_TRY(hipMalloc((void**)&L->md_partials,
+                              sizeof(double) * 2 * (size_t)md_sums_blocks(L, VAR_LINK_XCD) * kReduceSlots));
     } else if (sums) {
         HIP_TRY(launch_hamiltonian_sum(L, L->U[L->cur], L->E, L->result));
     }
@@ -1038,12 +1041,12 @@ int lqcd_hmc_trajectory(lqcd_lattice* L, double beta, double dt, size_t n, int d
     CHECK_ARG(drift == LQCD_DRIFT_ADDITIVE || drift == LQCD_DRIFT_EXP, "unknown drift mode");
     CHECK_ARG(scheme == LQCD_SCHEME_REFERENCE || scheme == LQCD_SCHEME_LEAPFROG, "unknown scheme");
     LATTICE_GUARD(L);
-    // The per-site MD kernels sum H_old's and H_new's terms on the way (the
+    // The MD kernels (md_variant_has_sums) sum H_old's and H_new's terms on the way (the
     // first launch over the starting links and momenta, the final kick over
     // the final ones; integrate_steps): every plaquette enters
     // sum Re Tr(U Sigma) through its 4 links, so
     // H_U = beta (N_plaquettes - sum Re Tr(U Sigma) / 12), H_E = beta sum e^2 / 2.
-    // Other work decompositions use the plaquette kernel before and after.
+    // Per-link kernels in f32 leave it to the plaquette kernel before and after.
     // Either way the sums stay on the device until the MD is done: one host
     // round trip per trajectory.
     int last = L->cur;

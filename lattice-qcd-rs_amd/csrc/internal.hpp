@@ -149,18 +149,22 @@ enum MdVariant {
 // VAR_SITE_TILE's LDS tile: whether it applies to the lattice, and its bytes
 bool md_tile_fits(const lqcd_lattice* L);
 size_t md_tile_bytes(const lqcd_lattice* L);
-// What an MD launch does besides its kick (+ drift).  Every variant: sums 3
-// (MdSums in md_device.hpp), the kick applied twice.  The per-site kernels
-// (variants 2-4): sums (0 none, 1 before the kick, 2 after it) of Re Tr(U Sigma) and e^2 into partials[block][0..1] (a
-// workgroup per 256 sites), and with two-row reads row 2 of the links read
-// written to row2 (null: not).
+// What an MD launch does besides its kick (+ drift).  sums (MdSums in
+// md_device.hpp): 0 none; 1 before the kick, 2 after it, of Re Tr(U Sigma) and
+// e^2 into partials[block][0..1] (md_sums_blocks workgroups); 3 no sums, the
+// kick applied twice.  row2, the per-site kernels with two-row reads: row 2 of
+// the links read is written there (null: not).
 struct MdExtra {
     int sums = 0;
     double* partials = nullptr;
     void* row2 = nullptr;
 };
-// whether an MD work decomposition takes MdExtra (the per-site kernels)
-bool md_variant_has_sums(int variant);
+// whether an MD work decomposition is per site (and takes MdExtra::row2)
+bool md_variant_per_site(int variant);
+// whether it sums the terms of H on the way (MdExtra::sums 1, 2)
+bool md_variant_has_sums(const lqcd_lattice* L, int variant);
+// workgroups (partials) of an MD launch with sums
+int64_t md_sums_blocks(const lqcd_lattice* L, int variant);
 hipError_t launch_kick_variant(const lqcd_lattice* L, int variant, const void* U, void* E, double kick,
                                const MdExtra* x = nullptr);
 hipError_t launch_kick_drift_variant(const lqcd_lattice* L, int variant, const void* U_in, void* U_out,

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_md(const vec2_t<S>* __restrict
         if (SITE)
             md_site<D, S, S, DR, R12, false, R01, TWICE ? KICK_TWICE : SUMS_NONE>(ui, uo, e, d.g, s, fs, (S)kick, df);
         else
-            md_link<D, S, S, DR, R12, R01, TWICE>(ui, uo, e, d.g, mu, s, fs, (S)kick, df);
+            md_link<D, S, S, DR, R12, R01, TWICE ? KICK_TWICE : SUMS_NONE>(ui, uo, e, d.g, mu, s, fs, (S)kick, df);
     }
 }
 

@@ -27,6 +27,8 @@
 //                 and the x_1 rows on either side, and reads the links one or
 //                 two steps away in x_0 / x_1 from LDS (20 of the 44 link
 //                 reads of a D = 4 site); the others come from U_in.
+#include <type_traits>
+
 #include "dispatch.hpp"
 #include "md_device.hpp"
 #include "observables_device.hpp"
@@ -118,31 +120,48 @@ __global__ __launch_bounds__(kBlock) void k_derivative_u(const vec2_t<S>* __rest
         }
 }
 
+// The per-link kernels sum in f64 fields only (md_variant_has_sums): in f32
+// their traces are f32 arithmetic, where the plaquette kernel's are f64.  Both
+// kernels put the partials of (mu, site block) at the same place, so H has the
+// same bits whichever of the two the autotuning takes.  An 8^4 f64 trajectory
+// of 20 steps is bound by the latency of its launches: without the plaquette
+// kernel and its reduction before and after the MD it takes 400 us, not 425.
+
 // VAR_LINK: grid (site blocks, D)
-template <int D, typename S, typename T, int DR, bool R12, bool TWICE>
+template <int D, typename S, typename T, int DR, bool R12, int FORM>
 __global__ __launch_bounds__(kBlock) void k_md_link(const vec2_t<S>* __restrict__ U_in,
                                                     vec2_t<S>* __restrict__ U_out,
                                                     S* __restrict__ E, Geom g, T fscale, T kick,
-                                                    T dfac)
+                                                    T dfac, double* __restrict__ partials)
 {
     const int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int mu = blockIdx.y;
-    if (s >= g.nsite) return;
-    md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP, TWICE>(U_in, U_out, E, g, mu, s, fscale, kick, dfac);
+    MdAcc<T> acc;
+    if (s < g.nsite)
+        md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP, FORM>(U_in, U_out, E, g, mu, s, fscale, kick, dfac, &acc);
+    if constexpr (md_sums(FORM)) {
+        double v[2] = {(double)acc.tr, (double)acc.e2};
+        block_reduce_to<2>(v, partials + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kReduceSlots);
+    }
 }
 
 // VAR_LINK_XCD: 1-D grid of (site block, mu) pairs, mu fastest, XCD remapped
-template <int D, typename S, typename T, int DR, bool R12, bool TWICE>
+template <int D, typename S, typename T, int DR, bool R12, int FORM>
 __global__ __launch_bounds__(kBlock) void k_md_link_xcd(const vec2_t<S>* __restrict__ U_in,
                                                         vec2_t<S>* __restrict__ U_out,
                                                         S* __restrict__ E, Geom g, T fscale, T kick,
-                                                        T dfac)
+                                                        T dfac, double* __restrict__ partials)
 {
     const int64_t logical = xcd_remap(blockIdx.x, gridDim.x);
     const int mu = (int)(logical % D);
     const int64_t s = (logical / D) * kBlock + threadIdx.x;
-    if (s >= g.nsite) return;
-    md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP, TWICE>(U_in, U_out, E, g, mu, s, fscale, kick, dfac);
+    MdAcc<T> acc;
+    if (s < g.nsite)
+        md_link<D, S, T, DR, R12, R12 && DR == DRIFT_EXP, FORM>(U_in, U_out, E, g, mu, s, fscale, kick, dfac, &acc);
+    if constexpr (md_sums(FORM)) {
+        double v[2] = {(double)acc.tr, (double)acc.e2};
+        block_reduce_to<2>(v, partials + (mu * (int64_t)(gridDim.x / D) + logical / D) * kReduceSlots);
+    }
 }
 
 // VAR_SITE_XCD / VAR_SITE_SLAB (slab_p > 0): one thread per site, all D links.
@@ -366,18 +385,27 @@ static void launch_md_variant_r(const lqcd_lattice* L, int variant, const void* 
             launch_site<D, S, DR, R12, SUMS_ON>(L, tile, nsb, ui, uo, e, fs, k, df, slab_p, slab_g, x);
         break;
     }
-    case VAR_LINK_XCD:
+    default: {
+        // per link: partials of the workgroups of all D directions
+        constexpr int SUMS_ON = DR >= 0 ? SUMS_BEFORE_KICK : SUMS_AFTER_KICK;
+        constexpr int TWICE_ON = DR >= 0 ? KICK_TWICE : SUMS_NONE;
+        double* partials = x ? x->partials : nullptr;
+        auto launch = [&](auto form) {
+            constexpr int FORM = decltype(form)::value;
+            if (variant == VAR_LINK_XCD)
+                k_md_link_xcd<D, S, S, DR, R12, FORM><<<nsb * (unsigned)D, kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df,
+                                                                                           partials);
+            else
+                k_md_link<D, S, S, DR, R12, FORM><<<link_grid(L), kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df, partials);
+        };
         if (twice)
-            k_md_link_xcd<D, S, S, DR, R12, DR >= 0><<<nsb * (unsigned)D, kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
+            launch(std::integral_constant<int, TWICE_ON>{});
+        else if (sizeof(S) == 8 && partials)
+            launch(std::integral_constant<int, sizeof(S) == 8 ? SUMS_ON : SUMS_NONE>{});
         else
-            k_md_link_xcd<D, S, S, DR, R12, false><<<nsb * (unsigned)D, kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
+            launch(std::integral_constant<int, SUMS_NONE>{});
         break;
-    default:
-        if (twice)
-            k_md_link<D, S, S, DR, R12, DR >= 0><<<link_grid(L), kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
-        else
-            k_md_link<D, S, S, DR, R12, false><<<link_grid(L), kBlock, 0, st>>>(ui, uo, e, L->g, fs, k, df);
-        break;
+    }
     }
 }
 
@@ -460,7 +488,17 @@ hipError_t launch_kick_drift(const lqcd_lattice* L, const void* U_in, void* U_ou
     return e;
 }
 
-bool md_variant_has_sums(int variant)
+int64_t md_sums_blocks(const lqcd_lattice* L, int variant)
+{
+    return (int64_t)grid_for(L->g.nsite) * (md_variant_per_site(variant) ? 1 : L->g.dim);
+}
+
+bool md_variant_has_sums(const lqcd_lattice* L, int variant)
+{
+    return md_variant_per_site(variant) || L->elem == 8;
+}
+
+bool md_variant_per_site(int variant)
 {
     return variant == VAR_SITE_XCD || variant == VAR_SITE_SLAB || variant == VAR_SITE_TILE;
 }

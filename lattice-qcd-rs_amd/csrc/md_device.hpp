@@ -364,39 +364,6 @@ __device__ __forceinline__ void kick_link(const T* f, T fscale, T kick, T* e)
     if constexpr (TWICE) kick_generators(f, kick * fscale, e);
 }
 
-// what happens with the force of one link (DR: -1 kick only, else drift mode)
-template <int DR, typename S, typename T, bool R01 = false, bool TWICE = false>
-__device__ __forceinline__ void finish_link(const mat3<T>& u, const mat3<T>& sigma,
-                                            vec2_t<S>* __restrict__ U_out, S* __restrict__ E,
-                                            const Geom& g, int mu, int64_t s, T fscale, T kick,
-                                            T dfac)
-{
-    mat3<T> m;
-    mul<false, false>(u, sigma, m);
-    T f[8], e[8];
-    im_trace_combinations(m, f);
-    load_e<T, S, kCacheStream>(E, g.npad, mu, s, e);
-    kick_link<TWICE>(f, fscale, kick, e);
-    store_e<T, S, kCacheStream>(E, g.npad, mu, s, e);
-    if constexpr (DR >= 0) drift_store<DR, R01, S, T>(u, e, dfac, U_out, g, mu, s);
-}
-
-// one link (mu, s): e += kick * F(U_in) (TWICE: two such kicks); U_out =
-// drift(U_in, e) unless DR < 0.
-// R12: links read as two rows (load_link_r12), for links in SU(3); R01: the
-// drifted link is stored as rows 0, 1 only.
-template <int D, typename S, typename T, int DR, bool R12 = false, bool R01 = false, bool TWICE = false>
-__device__ __forceinline__ void md_link(const vec2_t<S>* __restrict__ U_in, vec2_t<S>* __restrict__ U_out,
-                                        S* __restrict__ E, const Geom& g, int mu, int64_t s, T fscale,
-                                        T kick, T dfac)
-{
-    const Neighbours<D> nb = neighbours<D>(g, s);
-    mat3<T> sigma;
-    staple_sum<D, S, T, R12>(U_in, g, mu, s, nb, sigma);
-    const mat3<T> u = load_link_sel<R12, T, S>(U_in, g.npad, mu, s);
-    finish_link<DR, S, T, R01, TWICE>(u, sigma, U_out, E, g, mu, s, fscale, kick, dfac);
-}
-
 // The Hamiltonian sums a fused MD launch can produce on the way (SUMS): the
 // trace sum sum_mu Re Tr(U_mu(x) Sigma_mu(x)) of the links it reads (every
 // plaquette enters it through each of its 4 links, so it is 4 sum_P Re Tr P)
@@ -425,6 +392,43 @@ __device__ __forceinline__ T e_squares8(const T* e)
 #pragma unroll
     for (int a = 0; a < 8; ++a) q = fma(e[a], e[a], q);
     return q;
+}
+
+// what happens with the force of one link (DR: -1 kick only, else drift mode)
+// FORM: MdSums
+template <int DR, typename S, typename T, bool R01 = false, int FORM = SUMS_NONE>
+__device__ __forceinline__ void finish_link(const mat3<T>& u, const mat3<T>& sigma,
+                                            vec2_t<S>* __restrict__ U_out, S* __restrict__ E,
+                                            const Geom& g, int mu, int64_t s, T fscale, T kick,
+                                            T dfac, MdAcc<T>* acc = nullptr)
+{
+    mat3<T> m;
+    mul<false, false>(u, sigma, m);
+    T f[8], e[8];
+    im_trace_combinations(m, f);
+    load_e<T, S, kCacheStream>(E, g.npad, mu, s, e);
+    if constexpr (md_sums(FORM)) acc->tr += re_trace(m);
+    if constexpr (FORM == SUMS_BEFORE_KICK) acc->e2 += e_squares8<T>(e);
+    kick_link<FORM == KICK_TWICE>(f, fscale, kick, e);
+    if constexpr (FORM == SUMS_AFTER_KICK) acc->e2 += e_squares8<T>(e);
+    store_e<T, S, kCacheStream>(E, g.npad, mu, s, e);
+    if constexpr (DR >= 0) drift_store<DR, R01, S, T>(u, e, dfac, U_out, g, mu, s);
+}
+
+// one link (mu, s): e += kick * F(U_in) (KICK_TWICE: two such kicks); U_out =
+// drift(U_in, e) unless DR < 0.
+// R12: links read as two rows (load_link_r12), for links in SU(3); R01: the
+// drifted link is stored as rows 0, 1 only.
+template <int D, typename S, typename T, int DR, bool R12 = false, bool R01 = false, int FORM = SUMS_NONE>
+__device__ __forceinline__ void md_link(const vec2_t<S>* __restrict__ U_in, vec2_t<S>* __restrict__ U_out,
+                                        S* __restrict__ E, const Geom& g, int mu, int64_t s, T fscale,
+                                        T kick, T dfac, MdAcc<T>* acc = nullptr)
+{
+    const Neighbours<D> nb = neighbours<D>(g, s);
+    mat3<T> sigma;
+    staple_sum<D, S, T, R12>(U_in, g, mu, s, nb, sigma);
+    const mat3<T> u = load_link_sel<R12, T, S>(U_in, g.npad, mu, s);
+    finish_link<DR, S, T, R01, FORM>(u, sigma, U_out, E, g, mu, s, fscale, kick, dfac, acc);
 }
 
 // all D links of site s, sharing the staple loads.  SUMS: add to acc (see
