@@ -81,7 +81,7 @@ REALS_KICK_R12 = 28
 # k_md_site_tile<4, float, float, 1, 0> for variant 4; every branch counted, so an
 # upper bound of the executed count), and the issue rate of
 # the vector ALU: 256 CUs x 4 SIMDs x 2.4 GHz, one wave64 instruction per 4 cycles per SIMD
-VALU_PER_SITE = {(2, True): 6971, (3, True): 6971, (4, True): 7703, (2, False): 6842, (3, False): 6842}
+VALU_PER_SITE = {(2, True): 6974, (3, True): 6974, (4, True): 7688, (2, False): 6881, (3, False): 6881}
 VALU_WAVE_INSTR_PER_S = 256 * 4 * 2.4e9 / 4
 REALS_PLAQ = 18
 REALS_EENERGY = 8
