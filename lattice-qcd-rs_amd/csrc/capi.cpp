@@ -487,7 +487,7 @@ int lqcd_lattice_create(lqcd_ctx* ctx, int dim, const size_t* extent, double siz
     L->g.nsite = n;
     L->g.npad = (n + 255) / 256 * 256;
     // the device addresses the 9 planes of one direction with 32-bit offsets
-    if ((uint64_t)L->g.npad * 9 * 2 * L->elem > kMaxPlaneBytes) {
+    if (!direction_addressable(L->g.npad, L->elem)) {
         delete L;
         return fail(LQCD_ERR_UNSUPPORTED, "lattice too large: the link planes of one direction exceed 4 GiB");
     }

@@ -9,20 +9,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "limits.hpp"
+
 namespace lqcd {
-
-constexpr int kMaxDim = 4;
-// the field planes of one direction (9 link elements) span less than 2^32
-// bytes: the device addresses them with 32-bit offsets
-constexpr uint64_t kMaxPlaneBytes = 0xFFFFFFFFull;
-
-struct Geom {
-    int dim;
-    int extent[kMaxDim];
-    int64_t stride[kMaxDim];
-    int64_t nsite;   // number of sites
-    int64_t npad;    // row length of every SoA plane (>= nsite, multiple of 256)
-};
 
 // Offsets to the +dir and -dir neighbours of site s (periodic wrap).  Site
 // indices of one lattice fit in 31 bits (the device field access uses 32-bit

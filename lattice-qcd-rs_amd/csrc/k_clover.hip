@@ -82,7 +82,7 @@ __device__ __forceinline__ void clover_at(const vec2_t<S>* __restrict__ U, const
 
 // Link loaders: U_d(y) through a resource over the 9 planes of direction d
 // (uniform d), or through one resource over all 9 D planes (d may differ
-// between the lanes of a wave; the planes must span less than 4 GiB).
+// between the lanes of a wave; all_links_addressable).
 template <typename S>
 struct DirLinks {
     const vec2_t<S>* __restrict__ U;
@@ -442,7 +442,7 @@ hipError_t launch_clover_fields(const lqcd_lattice* L, int mode, double* d_out)
                                 (const vec2_t<S>*)L->U[L->cur], L->g, d_out, inv));
         break;
     case 1:
-        if ((uint64_t)L->g.npad * 9 * L->g.dim * L->elem <= kMaxPlaneBytes) {
+        if (all_links_addressable(L->g, L->elem)) {
             const unsigned nb = (unsigned)((L->g.nsite + 31) / 32);
             LQCD_DISPATCH_DS(L, k_f_mu_nu_blocks<D, S><<<nb, FPairs<D>::threads, 0, L->ctx->stream>>>(
                                     (const vec2_t<S>*)L->U[L->cur], L->g, d_out, inv));
