@@ -469,7 +469,8 @@ typedef enum {
     LQCD_KERNEL_FIELDS = 9,
     LQCD_KERNEL_STATS = 10,
     LQCD_KERNEL_HEAT_BATH = 11,
-    LQCD_KERNEL_OVERRELAX = 12
+    LQCD_KERNEL_OVERRELAX = 12,
+    LQCD_KERNEL_REORDER = 13 /* links between site and parity order */
 } lqcd_kernel_kind;
 
 /* ---------------------------------------------------------- statistics */

@@ -102,7 +102,8 @@ enum ProfileKind {
     PROF_STATS = 10,
     PROF_HEAT_BATH = 11,
     PROF_OVERRELAX = 12,
-    PROF_NKINDS = 13
+    PROF_REORDER = 13,
+    PROF_NKINDS = 14
 };
 
 // ---- fields (k_fields.hip) ----

@@ -574,12 +574,15 @@ __global__ __launch_bounds__(kBlock) void k_reorder_links(const vec2_t<S>* __res
 hipError_t launch_reorder_links(const lqcd_lattice* L, const void* in, void* out, bool to_parity)
 {
     const dim3 grid(grid_for(L->g.nsite), (unsigned)L->g.dim);
+    lqcd_prof_event ev;
+    prof_begin(L->ctx, PROF_REORDER, &ev);
     if (to_parity)
         LQCD_DISPATCH_DS(L, k_reorder_links<D, S, true><<<grid, kBlock, 0, L->ctx->stream>>>(
                                 (const vec2_t<S>*)in, (vec2_t<S>*)out, L->g));
     else
         LQCD_DISPATCH_DS(L, k_reorder_links<D, S, false><<<grid, kBlock, 0, L->ctx->stream>>>(
                                 (const vec2_t<S>*)in, (vec2_t<S>*)out, L->g));
+    prof_end(L->ctx, &ev);
     return hipGetLastError();
 }
 
