@@ -342,6 +342,7 @@ namespace lqcd {
 
 hipError_t site_order_links(lqcd_lattice* L)
 {
+    L->order.site_call();
     if (!L->parity_order) return hipSuccess;
     const int w = (L->cur + 1) % 3;
     const hipError_t e = launch_reorder_links(L, L->U[L->cur], L->U[w], false);
@@ -580,6 +581,7 @@ int lqcd_links_cold(lqcd_lattice* L)
 {
     CHECK_ARG(L, "lattice is null");
     DeviceGuard dg(L->ctx->device);
+    L->order.site_call();
     L->parity_order = false;   // every link is written
     HIP_TRY(launch_links_cold(L, L->U[L->cur]));
     HIP_TRY(hipStreamSynchronize(L->ctx->stream));
@@ -591,6 +593,7 @@ int lqcd_links_random(lqcd_lattice* L, uint64_t seed)
 {
     CHECK_ARG(L, "lattice is null");
     DeviceGuard dg(L->ctx->device);
+    L->order.site_call();
     L->parity_order = false;   // every link is written
     HIP_TRY(launch_links_random(L, L->U[L->cur], seed));
     HIP_TRY(hipStreamSynchronize(L->ctx->stream));
@@ -1107,21 +1110,30 @@ int lqcd_wilson_backward_device(lqcd_lattice* L, double beta, double* d_grad, si
     return LQCD_OK;
 }
 
-// Puts the links in parity order for the class launches of a sweep, where
-// that pays.  A class updates the sites of one parity, every other one of a
-// row: in site order its loads use half of each 128-byte line, and the other
-// half comes in again for the next staple.  f64 class launches at 32^4: heat
-// bath 328 -> 204 us, overrelaxation 325 -> 241, Metropolis 200 -> 137; D = 3
-// 128^3: 442 -> 295, 455 -> 377, 271 -> 209.  Reordering takes 265 us at 32^4, once: sweeps,
-// normalisation, plaquette and force read this order too, and other calls turn it
-// back (site_order_links).  Not for f32, where the launches gain 6-11 %, less than two
-// reorderings cost, nor for links that fit in the 32 MiB of the eight L2s
-// (12 x 14^3: 30.0 -> 26.7 us per launch, 16 us per reordering).
-constexpr size_t kParityOrderBytes = (size_t)32 << 20;
-
-static int class_order_links(lqcd_lattice* L)
+// The order of the links for a sweep.  A class updates the sites of one
+// parity, every other one of a row: in site order its loads use half of each
+// 128-byte line, and the other half comes in again for the next staple.  In
+// parity order f64 class launches take, at 32^4: heat bath 328 -> 204 us,
+// overrelaxation 325 -> 241, Metropolis 200 -> 137; D = 3 128^3: 442 -> 295,
+// 455 -> 377, 271 -> 209.  Sweeps, normalisation, plaquette and force read
+// either order (the last two up to 16 % slower in parity order: 32^4 212 ->
+// 246 and 561 -> 604 us); other calls turn it back (site_order_links).  When
+// that pays: sweep_order.hpp.  LQCD_SWEEP_ORDER=site or parity (f64 fields of
+// any size) pins the order.
+static int class_order_links(lqcd_lattice* L, SweepKind kind, size_t n_update)
 {
-    if (L->parity_order || L->precision != LQCD_F64 || L->nlink * 18 * L->elem < kParityOrderBytes) return LQCD_OK;
+    const double gain =
+        parity_order_gain(kind, L->precision == LQCD_F64, L->g.dim, L->nlink * 18 * L->elem, n_update);
+    bool parity = L->order.pays(gain);
+    L->order.swept(gain);
+    if (const char* env = std::getenv("LQCD_SWEEP_ORDER")) {
+        if (std::strcmp(env, "site") == 0) {
+            HIP_TRY(site_order_links(L));
+            return LQCD_OK;
+        }
+        if (std::strcmp(env, "parity") == 0) parity = L->precision == LQCD_F64;
+    }
+    if (L->parity_order || !parity) return LQCD_OK;
     const int w = (L->cur + 1) % 3;
     HIP_TRY(launch_reorder_links(L, L->U[L->cur], L->U[w], true));
     L->cur = w;
@@ -1169,7 +1181,7 @@ int lqcd_metropolis_sweep_random(lqcd_lattice* L, double beta, size_t n_update, 
         L->md_r12 = ok;
     }
     L->md_r12_last = L->md_r12;
-    if (int rc = class_order_links(L)) return rc;
+    if (int rc = class_order_links(L, SWEEP_METROPOLIS, n_update)) return rc;
     for (int mu = 0; mu < L->g.dim; ++mu)
         for (int par = 0; par < 2; ++par)
             HIP_TRY(launch_metropolis_class_rng(L, L->U[L->cur], mu, par, beta, n_update, spread, seed,
@@ -1190,7 +1202,7 @@ int lqcd_metropolis_sweep(lqcd_lattice* L, double beta, size_t n_update, const d
     HIP_TRY(hipMemcpyAsync(dp.p, proposals, pbytes, hipMemcpyHostToDevice, L->ctx->stream));
     HIP_TRY(hipMemcpyAsync(du.p, uniforms, sizeof(uint64_t) * L->nlink, hipMemcpyHostToDevice,
                            L->ctx->stream));
-    if (int rc = class_order_links(L)) return rc;
+    if (int rc = class_order_links(L, SWEEP_METROPOLIS, n_update)) return rc;
     for (int mu = 0; mu < L->g.dim; ++mu)
         for (int par = 0; par < 2; ++par)
             HIP_TRY(launch_metropolis_class(L, L->U[L->cur], mu, par, beta, n_update,
@@ -1225,7 +1237,7 @@ int lqcd_heat_bath_sweep(lqcd_lattice* L, double beta, uint64_t seed, uint64_t c
     CHECK_ARG(std::isfinite(beta) && beta > 0.0, "beta must be positive and finite");
     DeviceGuard dg(L->ctx->device);
     if (int rc = metropolis_prepare(L, beta, 1)) return rc;
-    if (int rc = class_order_links(L)) return rc;
+    if (int rc = class_order_links(L, SWEEP_HEAT_BATH, 1)) return rc;
     for (int mu = 0; mu < L->g.dim; ++mu)
         for (int par = 0; par < 2; ++par)
             HIP_TRY(launch_heat_bath_class(L, L->U[L->cur], mu, par, beta, seed, counter));
@@ -1243,7 +1255,7 @@ static int overrelaxation(lqcd_lattice* L, bool reverse)
     for (int i = 0; i < L->g.dim; ++i)
         if (L->g.extent[i] % 2) return fail(LQCD_ERR_UNSUPPORTED, "checkerboard sweep needs even extents");
     DeviceGuard dg(L->ctx->device);
-    if (int rc = class_order_links(L)) return rc;
+    if (int rc = class_order_links(L, SWEEP_OVERRELAX, 1)) return rc;
     for (int mu = 0; mu < L->g.dim; ++mu)
         for (int par = 0; par < 2; ++par) HIP_TRY(launch_overrelax_class(L, L->U[L->cur], mu, par, reverse));
     HIP_TRY(hipStreamSynchronize(L->ctx->stream));

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "geometry.hpp"
+#include "sweep_order.hpp"
 
 struct lqcd_prof_event {
     int kind;
@@ -40,6 +41,7 @@ struct lqcd_lattice {
     // the f64 checkerboard sweeps, undone by site_order_links before anything
     // that reads them in site order
     bool parity_order = false;
+    lqcd::SweepOrder order;  // when they are put there
     void* E = nullptr;
     double* partials = nullptr;  // per-block reduction scratch
     double* result = nullptr;    // device reduction results
