@@ -552,12 +552,13 @@ int lqcd_links_upload(lqcd_lattice* L, const double* links, size_t n_links)
 {
     CHECK_ARG(L && links, "null argument");
     if (int rc = check_links(L, n_links)) return rc;
-    LATTICE_GUARD(L);
+    DeviceGuard dg(L->ctx->device);
     DevBuf st;
     HIP_TRY(hipMalloc(&st.p, sizeof(double) * 18 * L->nlink));
     HIP_TRY(hipMemcpyAsync(st.p, links, sizeof(double) * 18 * L->nlink, hipMemcpyHostToDevice,
                            L->ctx->stream));
     HIP_TRY(launch_links_from_aos(L, (const double*)st.p, L->U[L->cur]));
+    links_replaced(L);
     HIP_TRY(hipStreamSynchronize(L->ctx->stream));
     L->su3_known = -1;
     return LQCD_OK;
@@ -581,9 +582,8 @@ int lqcd_links_cold(lqcd_lattice* L)
 {
     CHECK_ARG(L, "lattice is null");
     DeviceGuard dg(L->ctx->device);
-    L->order.site_call();
-    L->parity_order = false;   // every link is written
     HIP_TRY(launch_links_cold(L, L->U[L->cur]));
+    links_replaced(L);
     HIP_TRY(hipStreamSynchronize(L->ctx->stream));
     L->su3_known = 0;
     return LQCD_OK;
@@ -593,9 +593,8 @@ int lqcd_links_random(lqcd_lattice* L, uint64_t seed)
 {
     CHECK_ARG(L, "lattice is null");
     DeviceGuard dg(L->ctx->device);
-    L->order.site_call();
-    L->parity_order = false;   // every link is written
     HIP_TRY(launch_links_random(L, L->U[L->cur], seed));
+    links_replaced(L);
     HIP_TRY(hipStreamSynchronize(L->ctx->stream));
     L->su3_known = 0;
     return LQCD_OK;

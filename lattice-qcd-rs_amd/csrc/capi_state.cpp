@@ -705,7 +705,7 @@ int read_bincode_into(lqcd_lattice* L, const char* path, int with_e, double* bet
             return fail(LQCD_ERR_INCOMPATIBLE_SIZE, "the state's lattice does not match the handle's extents");
     if (b.size != L->size)
         return fail(LQCD_ERR_INCOMPATIBLE_SIZE, "the state's lattice spacing does not match the handle's");
-    LATTICE_GUARD(L);
+    DeviceGuard dg(L->ctx->device);
     hipStream_t s = L->ctx->stream;
     const uint64_t ne = with_e ? (uint64_t)L->nlink * 64 : 0, nl = (uint64_t)L->nlink * 144;
     DevBuf stage;
@@ -720,6 +720,7 @@ int read_bincode_into(lqcd_lattice* L, const char* path, int with_e, double* bet
     }
     // the whole file is in HBM: only now is the lattice overwritten
     HIP_TRY(launch_links_from_aos(L, (const double*)(d + ne), L->U[L->cur]));
+    links_replaced(L);
     if (with_e) HIP_TRY(launch_efield_from_aos(L, (const double*)d, L->E));
     HIP_TRY(hipStreamSynchronize(s));
     L->su3_known = -1;

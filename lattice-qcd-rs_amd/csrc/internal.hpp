@@ -197,6 +197,13 @@ hipError_t launch_metropolis_class_rng(const lqcd_lattice* L, void* U, int mu, i
 hipError_t launch_reorder_links(const lqcd_lattice* L, const void* in, void* out, bool to_parity);
 // the lattice's current links back in site order (enqueued; capi.cpp)
 hipError_t site_order_links(lqcd_lattice* L);
+// every link of the current buffer has been overwritten in site order
+// (enqueued; until then the links keep the order they have)
+inline void links_replaced(lqcd_lattice* L)
+{
+    L->order.site_call();
+    L->parity_order = false;
+}
 // heat bath / overrelaxation of one (mu, parity) class (k_mc.hip); the heat
 // bath writes the per-link count of exhausted samplers to mh_acc (mh_p = 0)
 hipError_t launch_heat_bath_class(const lqcd_lattice* L, void* U, int mu, int parity, double beta, uint64_t seed,
