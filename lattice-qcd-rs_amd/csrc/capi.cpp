@@ -1114,8 +1114,8 @@ int lqcd_wilson_backward_device(lqcd_lattice* L, double beta, double* d_grad, si
 // 128-byte line, and the other half comes in again for the next staple.  In
 // parity order f64 class launches take, at 32^4: heat bath 328 -> 204 us,
 // overrelaxation 325 -> 241, Metropolis 200 -> 137; D = 3 128^3: 442 -> 295,
-// 455 -> 377, 271 -> 209.  Sweeps, normalisation, plaquette and force read
-// either order (the last two up to 16 % slower in parity order: 32^4 212 ->
+// 455 -> 377, 271 -> 209.  Sweeps, link updates, normalisation, plaquette and force read
+// either order (the last two up to 19 % slower in parity order: 32^4 212 ->
 // 246 and 561 -> 604 us); other calls turn it back (site_order_links).  When
 // that pays: sweep_order.hpp.  LQCD_SWEEP_ORDER=site or parity (f64 fields of
 // any size) pins the order.
@@ -1218,7 +1218,7 @@ int lqcd_metropolis_link_random(lqcd_lattice* L, double beta, double spread, uin
     CHECK_ARG(std::isfinite(beta), "beta must be finite");
     // MetropolisHastingsDeltaDiagnostic::new returns None outside (0, 1)
     CHECK_ARG(spread > 0.0 && spread < 1.0, "spread must be in (0, 1)");
-    LATTICE_GUARD(L);
+    DeviceGuard dg(L->ctx->device);
     HIP_TRY(launch_metropolis_link(L, L->U[L->cur], beta, spread, seed, counter, L->result));
     if (int rc = read_results(L, 3)) return rc;
     if (probability) *probability = L->host_result[0];

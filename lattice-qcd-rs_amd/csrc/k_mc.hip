@@ -214,7 +214,7 @@ __global__ __launch_bounds__(kBlock) void k_metropolis(vec2_t<S>* __restrict__ U
 // block 62 of link 0 (site = (x y) * nsite >> 64 over the 64-bit word of
 // x, y; direction = z * D >> 32), then the proposal and accept word of that
 // link as in the device sweep.  One lane works; out = p, accepted, link.
-template <int D, typename S>
+template <int D, typename S, bool PO>
 __global__ __launch_bounds__(64) void k_metropolis_link(vec2_t<S>* __restrict__ U, Geom g, double beta,
                                                         double spread, uint64_t seed, uint64_t counter,
                                                         double* __restrict__ out)
@@ -225,8 +225,10 @@ __global__ __launch_bounds__(64) void k_metropolis_link(vec2_t<S>* __restrict__ 
     const int64_t s = (int64_t)__umul64hi(w, (uint64_t)g.nsite);
     const int mu = (int)(((uint64_t)o.z * (uint64_t)D) >> 32);
     mat3<double> a, r, nw;
-    mc_staple<D, S>(U, g, mu, s, SiteMap<D, false>(g, 0), a);
-    const mat3<double> u = load_link<double, S>(U, g.npad, mu, s);
+    const SiteMap<D, PO> sm(g, s);
+    const int64_t own = sm.template at<0>(s);
+    mc_staple<D, S, false, PO>(U, g, mu, s, sm, a);
+    const mat3<double> u = load_link<double, S>(U, g.npad, mu, own);
     const int64_t li = s * D + mu;
     device_proposal((uint64_t)li, 0, seed, counter, spread, r);
     mul<false, false>(r, u, nw);
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(64) void k_metropolis_link(vec2_t<S>* __restrict__ 
     out[0] = p;
     out[1] = accept ? 1.0 : 0.0;
     out[2] = (double)li;
-    if (accept) store_link<double, S>(U, g.npad, mu, s, nw);
+    if (accept) store_link<double, S>(U, g.npad, mu, own, nw);
 }
 
 // ---------------------------------------------------------------- heat bath
@@ -640,7 +642,7 @@ hipError_t launch_metropolis_class(const lqcd_lattice* L, void* U, int mu, int p
 hipError_t launch_metropolis_link(const lqcd_lattice* L, void* U, double beta, double spread, uint64_t seed,
                                   uint64_t counter, double* d_out3)
 {
-    LQCD_DISPATCH_DS(L, k_metropolis_link<D, S><<<1, 64, 0, L->ctx->stream>>>(
+    LQCD_DISPATCH_DS_PO(L, k_metropolis_link<D, S, PO><<<1, 64, 0, L->ctx->stream>>>(
                             (vec2_t<S>*)U, L->g, beta, spread, seed, counter, d_out3));
     return hipGetLastError();
 }
