@@ -16,6 +16,7 @@
 #include "capi_util.hpp"
 #include "dispatch.hpp"
 #include "internal.hpp"
+#include "optional_buffers.hpp"
 
 using namespace lqcd;
 
@@ -656,6 +657,19 @@ static int ensure_gauss_buffers(lqcd_lattice* L)
     return LQCD_OK;
 }
 
+// the projection's transports; false where their memory cannot be had: the
+// projection then takes the steps without them
+static bool ensure_gauss_transports(lqcd_lattice* L)
+{
+    auto alloc = [](double** p, size_t bytes) {
+        if (hipMalloc((void**)p, bytes) == hipSuccess) return true;
+        (void)hipGetLastError();   // or the next launch would report it
+        return false;
+    };
+    return both_or_neither(L->gauss_t, sizeof(double) * 9 * (size_t)L->g.npad * L->g.dim, alloc,
+                           [](double* p) { (void)hipFree(p); });
+}
+
 int lqcd_efield_gauss(lqcd_lattice* L, double* out, size_t n_sites)
 {
     CHECK_ARG(L && out, "null argument");
@@ -759,12 +773,8 @@ int lqcd_efield_project_gauss(lqcd_lattice* L, size_t max_iter, size_t* iteratio
     // other than the checked field, which stays the result if the check passes.
     double* const buf[3] = {L->gauss_e[0], L->gauss_e[1], L->gauss_e[2]};
     double* tr[2] = {nullptr, nullptr};   // transports; tr[1] goes with buf[cur] at a check
-    if (gauss_uses_transports(L))
-        for (int k = 0; k < 2; ++k) {
-            if (!L->gauss_t[k])
-                HIP_TRY(hipMalloc((void**)&L->gauss_t[k], sizeof(double) * 9 * (size_t)L->g.npad * L->g.dim));
-            tr[k] = L->gauss_t[k];
-        }
+    if (gauss_uses_transports(L) && ensure_gauss_transports(L))
+        for (int k = 0; k < 2; ++k) tr[k] = L->gauss_t[k];
     int cur = 1;
     HIP_TRY(launch_gauss_start(L, buf[0], tr[0]));
     HIP_TRY(launch_gauss_step(L, buf[0], tr[0], buf[1], tr[1], nullptr));
