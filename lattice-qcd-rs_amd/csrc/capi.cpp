@@ -15,6 +15,7 @@
 #include "../../include/lqcd.h"
 #include "capi_util.hpp"
 #include "dispatch.hpp"
+#include "gauss_rules.hpp"
 #include "internal.hpp"
 #include "optional_buffers.hpp"
 
@@ -773,7 +774,7 @@ int lqcd_efield_project_gauss(lqcd_lattice* L, size_t max_iter, size_t* iteratio
     // other than the checked field, which stays the result if the check passes.
     double* const buf[3] = {L->gauss_e[0], L->gauss_e[1], L->gauss_e[2]};
     double* tr[2] = {nullptr, nullptr};   // transports; tr[1] goes with buf[cur] at a check
-    if (gauss_uses_transports(L) && ensure_gauss_transports(L))
+    if (gauss_uses_transports(L->g) && ensure_gauss_transports(L))
         for (int k = 0; k < 2; ++k) tr[k] = L->gauss_t[k];
     int cur = 1;
     HIP_TRY(launch_gauss_start(L, buf[0], tr[0]));

@@ -73,9 +73,7 @@ struct lqcd_lattice {
 
 namespace lqcd {
 
-constexpr int kBlock = 256;
 constexpr int kReduceSlots = 4;   // doubles per block partial
-constexpr int kMaxReduceBlocks = 4096;
 // device Metropolis proposals use Philox blocks 64 + 8 j + (0..6), below the
 // heat-bath blocks (32768..)
 constexpr size_t kMaxMhUpdates = 4000;
@@ -226,8 +224,6 @@ hipError_t launch_plaquette_field(const lqcd_lattice* L, int which, int a, bool 
 // G(x) of the double E copy Ed, and div = sum_x |Tr(sum_a T^a G(x))| into d_div
 hipError_t launch_gauss(const lqcd_lattice* L, const double* Ed, double* d_div);
 hipError_t launch_gauss_to_aos(const lqcd_lattice* L, double* d_out);
-// whether the projection's steps carry the transports U^+ E U of E along
-bool gauss_uses_transports(const lqcd_lattice* L);
 // E to its double copy Ed, and its transports to T (9 npad doubles per
 // direction; null: steps without them)
 hipError_t launch_gauss_start(const lqcd_lattice* L, double* Ed, double* T);

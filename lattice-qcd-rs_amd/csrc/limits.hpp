@@ -1,5 +1,6 @@
-// limits.hpp -- lattice geometry and the sizes the device can address: plain
-// C++, so that the choices made from them can be checked without a device.
+// limits.hpp -- lattice geometry, the sizes the device can address and those of
+// launches: plain C++, so that the choices made from them can be checked without
+// a device.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
@@ -7,6 +8,10 @@
 namespace lqcd {
 
 constexpr int kMaxDim = 4;
+// threads of a workgroup, where a kernel has no number of its own, and the most
+// workgroups of a reduction
+constexpr int kBlock = 256;
+constexpr int kMaxReduceBlocks = 4096;
 // the planes behind one buffer resource span less than 2^32 bytes: the device
 // addresses them with 32-bit offsets
 constexpr uint64_t kMaxPlaneBytes = 0xFFFFFFFFull;
