@@ -442,11 +442,11 @@ __global__ __launch_bounds__(kBlock) void k_gauss_start(const vec2_t<S>* __restr
 
 // One project_to_gauss_step of the whole field, E_in, T_in -> E_out, T_out,
 // and the block partials of div(E_in).  Bound by latency on the lattices that
-// take it (gauss_uses_transports): no G is evaluated by products, and all
-// loads of a link are issued before the barrier (16^4 f64 28.7 -> 27.7 us, 8^4
-// 10.4 -> 8.5).  A workgroup takes `chunk` consecutive
-// tiles of 64 sites, one link of a site per thread (wave i: direction i): the
-// waves' terms of G(x) meet in LDS, each wave forms G(x + i) itself.
+// take it (gauss_uses_transports, D = 2 and 4): no G is evaluated by products,
+// and all loads of a link are issued before the barrier (8^4 f64 10.4 -> 8.5 us
+// per step).  A workgroup takes `chunk` consecutive tiles of 64 sites, one link
+// of a site per thread (wave i: direction i): the waves' terms of G(x) meet in
+// LDS, each wave forms G(x + i) itself.
 template <int D, typename S>
 __global__ __launch_bounds__(64 * D) void k_gauss_links(const vec2_t<S>* __restrict__ U, const double* __restrict__ E_in,
                                                         const double* __restrict__ T_in, Geom g,
@@ -766,7 +766,8 @@ hipError_t launch_gauss_start(const lqcd_lattice* L, double* Ed, double* T)
 {
     if (!T) return launch_efield_to_double(L, L->E, Ed);
     const dim3 grid(grid_for(L->g.nsite), (unsigned)L->g.dim);
-    LQCD_DISPATCH_DS(L, k_gauss_start<D, S><<<grid, kBlock, 0, L->ctx->stream>>>(
+    if (L->g.dim == 3) return hipErrorInvalidValue;   // gauss_uses_transports: not built
+    LQCD_DISPATCH_DS(L, if constexpr (D != 3) k_gauss_start<D, S><<<grid, kBlock, 0, L->ctx->stream>>>(
                             (const vec2_t<S>*)L->U[L->cur], (const S*)L->E, L->g, Ed, T));
     return hipGetLastError();
 }
@@ -778,10 +779,11 @@ hipError_t launch_gauss_step(const lqcd_lattice* L, const double* E_in, const do
     hipStream_t st = L->ctx->stream;
     int nb;
     if (T_in) {
+        if (L->g.dim == 3) return hipErrorInvalidValue;
         const int64_t tiles = (L->g.nsite + 63) / 64;
         const int chunk = (int)((tiles + kMaxReduceBlocks - 1) / kMaxReduceBlocks);
         nb = (int)((tiles + chunk - 1) / chunk);
-        LQCD_DISPATCH_DS(L, k_gauss_links<D, S><<<nb, 64 * D, 0, st>>>((const vec2_t<S>*)U, E_in, T_in, L->g, E_out,
+        LQCD_DISPATCH_DS(L, if constexpr (D != 3) k_gauss_links<D, S><<<nb, 64 * D, 0, st>>>((const vec2_t<S>*)U, E_in, T_in, L->g, E_out,
                                                                         T_out, L->partials, chunk));
     } else if (const GaussTiles gt = gauss_tiles(L->g); gt.a > 0) {
         nb = gt.nblocks;
