@@ -172,7 +172,7 @@ static hipError_t launch_md_step(lqcd_lattice* L, int src, int dst, double dt, s
 {
     const bool ref = scheme == LQCD_SCHEME_REFERENCE;
     MdExtra two;
-    two.sums = 3;
+    two.sums = KICK_TWICE;
     return launch_kick_drift(L, L->U[src], L->U[dst], L->E, k == 0 || ref ? dt / 2.0 : dt, dt, drift,
                              k > 0 && ref ? &two : x);
 }
@@ -291,9 +291,9 @@ int integrate_steps(lqcd_lattice* L, double dt, size_t n, int drift, int scheme,
     const int final_buf = buffer_after(L, n);
     MdExtra first, fin;
     if (with_sums) {
-        first.sums = 1;
+        first.sums = SUMS_BEFORE_KICK;
         first.partials = L->md_partials;
-        fin.sums = 2;
+        fin.sums = SUMS_AFTER_KICK;
         fin.partials = L->md_partials + nb * kReduceSlots;
     }
     // the final kick reads the final links as two rows and completes them

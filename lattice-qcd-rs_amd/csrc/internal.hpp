@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "geometry.hpp"
+#include "md_form.hpp"
 #include "sweep_order.hpp"
 
 struct lqcd_prof_event {
@@ -150,19 +151,18 @@ enum MdVariant {
 // VAR_SITE_TILE's LDS tile: whether it applies to the lattice, and its bytes
 bool md_tile_fits(const lqcd_lattice* L);
 size_t md_tile_bytes(const lqcd_lattice* L);
-// What an MD launch does besides its kick (+ drift).  sums (MdSums in
-// md_device.hpp): 0 none; 1 before the kick, 2 after it, of Re Tr(U Sigma) and
-// e^2 into partials[block][0..1] (md_sums_blocks workgroups); 3 no sums, the
-// kick applied twice.  row2, the per-site kernels with two-row reads: row 2 of
-// the links read is written there (null: not).
+// What an MD launch does besides its kick (+ drift): sums, its form (MdSums in
+// md_form.hpp), with the sums of Re Tr(U Sigma) and e^2 in partials[block][0..1]
+// (md_sums_blocks workgroups); row2, the per-site kernels with two-row reads:
+// row 2 of the links read is written there (null: not).
 struct MdExtra {
-    int sums = 0;
+    int sums = SUMS_NONE;
     double* partials = nullptr;
     void* row2 = nullptr;
 };
 // whether an MD work decomposition is per site (and takes MdExtra::row2)
 bool md_variant_per_site(int variant);
-// whether it sums the terms of H on the way (MdExtra::sums 1, 2)
+// whether it sums the terms of H on the way (md_sums)
 bool md_variant_has_sums(const lqcd_lattice* L, int variant);
 // workgroups (partials) of an MD launch with sums
 int64_t md_sums_blocks(const lqcd_lattice* L, int variant);

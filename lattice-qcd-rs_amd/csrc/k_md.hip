@@ -400,10 +400,10 @@ static void launch_md_variant_r(const lqcd_lattice* L, int variant, const void* 
         };
         if (twice)
             launch(std::integral_constant<int, TWICE_ON>{});
-        else if (sizeof(S) == 8 && partials)
-            launch(std::integral_constant<int, sizeof(S) == 8 ? SUMS_ON : SUMS_NONE>{});
-        else
+        else if (sums == SUMS_NONE)
             launch(std::integral_constant<int, SUMS_NONE>{});
+        else
+            launch(std::integral_constant<int, sizeof(S) == 8 ? SUMS_ON : SUMS_NONE>{});
         break;
     }
     }
@@ -449,9 +449,17 @@ hipError_t launch_force_store(const lqcd_lattice* L, const void* U, double* d_ou
     return hipGetLastError();
 }
 
+// x->sums alone chooses the form; a launch that is not built in it, or has no
+// partials to write its sums to, is refused
+static bool extra_valid(const lqcd_lattice* L, int variant, bool drift, const MdExtra* x)
+{
+    return !x || md_form_valid(x->sums, drift, md_variant_has_sums(L, variant), x->partials != nullptr);
+}
+
 hipError_t launch_kick_variant(const lqcd_lattice* L, int variant, const void* U, void* E, double kick,
                                const MdExtra* x)
 {
+    if (!extra_valid(L, variant, false, x)) return hipErrorInvalidValue;
     LQCD_DISPATCH_DS(L, launch_md_variant<D, S, -1>(L, variant, U, nullptr, E, kick, 0.0, x));
     return hipGetLastError();
 }
@@ -459,6 +467,7 @@ hipError_t launch_kick_variant(const lqcd_lattice* L, int variant, const void* U
 hipError_t launch_kick_drift_variant(const lqcd_lattice* L, int variant, const void* U_in, void* U_out,
                                      void* E, double kick, double dt, int drift_mode, const MdExtra* x)
 {
+    if (!extra_valid(L, variant, true, x)) return hipErrorInvalidValue;
     const double df = md_drift_scale(dt, L->size);
     if (drift_mode == DRIFT_EXP) {
         LQCD_DISPATCH_DS(L, launch_md_variant<D, S, DRIFT_EXP>(L, variant, U_in, U_out, E, kick, df, x));

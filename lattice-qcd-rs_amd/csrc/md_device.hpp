@@ -364,15 +364,8 @@ __device__ __forceinline__ void kick_link(const T* f, T fscale, T kick, T* e)
     if constexpr (TWICE) kick_generators(f, kick * fscale, e);
 }
 
-// The Hamiltonian sums a fused MD launch can produce on the way (SUMS): the
-// trace sum sum_mu Re Tr(U_mu(x) Sigma_mu(x)) of the links it reads (every
-// plaquette enters it through each of its 4 links, so it is 4 sum_P Re Tr P)
-// and the momentum sum sum_mu,a e^a_mu(x)^2 of E before the kick
-// (SUMS_BEFORE_KICK: the first launch of a trajectory, H_old) or after it
-// (SUMS_AFTER_KICK: the final kick, H_new); accumulated per thread in double.
-// KICK_TWICE is the fourth form of a launch: no sums, two kicks (kick_link).
-enum MdSums { SUMS_NONE = 0, SUMS_BEFORE_KICK = 1, SUMS_AFTER_KICK = 2, KICK_TWICE = 3 };
-__host__ __device__ constexpr bool md_sums(int form) { return form == SUMS_BEFORE_KICK || form == SUMS_AFTER_KICK; }
+// a thread's terms of the sums of a launch (MdSums), in the kernel's arithmetic;
+// they are added over the threads in double
 template <typename T>
 struct MdAcc {
     T tr = T(0);
