@@ -29,10 +29,11 @@ constexpr int kGaussHaloMax = kBlock;
 // (or LQCD_GAUSS_TILES=0 pins the site walk): L0 divides 64 (whole x_0 rows
 // per wavefront), a tile L0 x a x b of kBlock sites with the rows of a
 // wavefront in one x_2 layer, a | L1, b | L2 and the smallest halo L0 (a + b);
-// C | L3 the largest of 32, 16, .., 1 that leaves min(512, the tiles of the
-// lattice) workgroups or more (512: one round of two workgroups per CU) and at
-// most kMaxReduceBlocks.  (With half the tiles as the floor the 256 tiles of 16^4
-// ran as 128 workgroups of C = 2, half the CUs: 34.4 against 29.3 us per f64 step.)
+// C | L3 the largest of 32, 16, .., 1 that leaves `target` workgroups or more and
+// at most kMaxReduceBlocks: 512 (one round of two per CU), or half of the tiles
+// where those are fewer than 1024, as C = 2 saves a quarter of the G evaluations
+// (the 512 tiles of 16^3 x 32, us per step of C = 1 -> 2: f64 60.5 -> 50.2, f32 42.0 -> 38.4), but not
+// below one workgroup per CU (the 256 tiles of 16^4, C = 1 -> 2: f64 29.3 -> 34.4).
 inline GaussTiles gauss_tiles(const Geom& g)
 {
     GaussTiles gt;
@@ -54,7 +55,8 @@ inline GaussTiles gauss_tiles(const Geom& g)
     if (best_a == 0) return gt;
     const int64_t tiles = (int64_t)(L1 / best_a) * (L2 / best_b);
     const int64_t all = tiles * L3;
-    const int64_t target = all < 512 ? all : 512;
+    const int64_t half = all / 2 < 512 ? all / 2 : 512;
+    const int64_t target = half > 256 ? half : all < 256 ? all : 256;
     int C = 0;
     for (int c : {32, 16, 8, 4, 2, 1})
         if (L3 % c == 0 && all / c >= target && all / c <= kMaxReduceBlocks) {

@@ -54,6 +54,7 @@ def rules(tmp_path_factory):
 CASES = [([8, 16, 8, 4], "transports", 1, "walk", "transports"), ([16, 8, 8, 4], "transports", 1, "walk", "transports"),
          ([8, 8, 4, 4], "transports", 1, "walk", "transports"), ([8] * 4, "transports", 1, "walk", "transports"),
          ([16, 16, 16, 8], 1, 1, "walk", "transports"), ([16] * 4, 1, 1, "walk", "transports"),
+         ([16, 16, 16, 32], 2, 2, "walk", "transports"), ([32, 16, 16, 16], 2, 2, "walk", "transports"),
          ([16, 16, 16, 64], 2, 2, "walk", "transports"), ([32, 16, 16, 32], 2, 2, "walk", "transports"),
          ([64, 16, 32, 16], 4, 4, "walk", "transports"), ([16, 16, 16, 128], 4, 4, "walk", "transports"),
          ([32] * 4, 8, 8, "walk", "transports"), ([12, 10, 6, 9], "transports", "walk", "walk", "transports"),
