@@ -4,8 +4,9 @@
 // x, word after word, so that a wavefront over 64 consecutive sites reads
 // 1 KiB in one fully coalesced request with 16 bytes per lane.
 //   links, f64: per direction 9 planes, entry k = row * 3 + col as (re, im);
-//   links, f32: per direction 4 planes of entry pairs (2p, 2p + 1) as (re, im,
-//               re, im), then a plane of 8-byte words with entry 8;
+//   links, f32: per direction 4 planes of entry pairs (0, 1), (3, 4), (2, 5),
+//               (6, 7) as (re, im, re, im), then a plane of 8-byte words with
+//               entry 8;
 //   E, f64:     per direction 4 planes of components (2w, 2w + 1);
 //   E, f32:     per direction 2 planes of components (4w .. 4w + 3).
 // Planes have g.npad words.  The words are 16 bytes because the vector L1
@@ -91,9 +92,15 @@ __device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, uint32_t off
     }
 }
 
-// Byte offset of link entry k of site `s` within a direction's planes, as a
-// per-lane part and a uniform part, for an access that starts at entry k
-// (f32: k even, or 8).
+// The f32 pairs are chosen so that the parts of a link that kernels read or write
+// alone are whole words: rows 0 and 1 (the two-row reads and stores) are pairs
+// 0-2, columns 0 and 1 (the normalisation) pairs 0, 1 and 3.  With pairs of
+// consecutive entries the normalisation read four words for three: us, 2048^2
+// 231 -> 198, 128^3 171 -> 148, 32^4 89 -> 77; the per-site kernels with additive
+// drift on small D = 3 lattices gained too (25x17x31 17.8 -> 12.5).
+
+// Byte offset of f64 entry k, f32 pair k / 2 or the last f32 entry (k = 8) of
+// site `s` within a direction's planes, as a per-lane part and a uniform part.
 template <typename S>
 __device__ __forceinline__ uint32_t link_off(int64_t s, int k)
 {
@@ -105,22 +112,37 @@ __device__ __forceinline__ uint32_t link_plane(int64_t npad, int k)
     return (uint32_t)k * (uint32_t)npad * 2u * (uint32_t)sizeof(S);
 }
 
+// Calls f(pair, entry, entry) for the f32 pairs of entries [K0, K1): all, rows 0
+// and 1 (K0 = 0, K1 = 6) or row 2's first two (K0 = 6).  Both parts of a link that a
+// kernel reads or writes alone are whole pairs: rows 0 and 1 (the two-row
+// reads and stores) pairs 0-2, columns 0 and 1 (the normalisation) pairs 0, 1 and 3.
+// With pairs of consecutive entries the normalisation read a third more than it
+// needs: XXNORM.
 // entries [K0, K1) of the link at byte offset `base` (per lane) of resource r
 template <int K0, int K1, typename T, typename S, int CP>
 __device__ __forceinline__ void load_entries(__amdgpu_buffer_rsrc_t r, uint32_t base, int64_t npad, int64_t s,
                                              mat3<T>& m)
 {
     if constexpr (sizeof(S) == 4) {
-        static_assert(K0 % 2 == 0 && (K1 % 2 == 0 || K1 == 9), "f32 links are read in pairs of entries");
-#pragma unroll
-        for (int k = K0; k + 1 < K1; k += 2) {
-            const float4 v = buf_load<float4, CP>(r, base + link_off<S>(s, k), link_plane<S>(npad, k));
-            m.e[k] = {T(v.x), T(v.y)};
-            m.e[k + 1] = {T(v.z), T(v.w)};
+        static_assert((K0 == 0 || K0 == 6) && (K1 == 6 || K1 == 9), "f32 links are read in whole pairs");
+        const uint32_t off = base + link_off<S>(s, 0);
+        if constexpr (K0 == 0) {
+            const float4 p = buf_load<float4, CP>(r, off, link_plane<S>(npad, 0));
+            const float4 q = buf_load<float4, CP>(r, off, link_plane<S>(npad, 2));
+            const float4 t = buf_load<float4, CP>(r, off, link_plane<S>(npad, 4));
+            m.e[0] = {T(p.x), T(p.y)};
+            m.e[1] = {T(p.z), T(p.w)};
+            m.e[2] = {T(t.x), T(t.y)};
+            m.e[3] = {T(q.x), T(q.y)};
+            m.e[4] = {T(q.z), T(q.w)};
+            m.e[5] = {T(t.z), T(t.w)};
         }
         if constexpr (K1 == 9) {
-            const float2 v = buf_load<float2, CP>(r, base + link_off<S>(s, 8), link_plane<S>(npad, 8));
-            m.e[8] = {T(v.x), T(v.y)};
+            const float4 p = buf_load<float4, CP>(r, off, link_plane<S>(npad, 6));
+            const float2 q = buf_load<float2, CP>(r, base + link_off<S>(s, 8), link_plane<S>(npad, 8));
+            m.e[6] = {T(p.x), T(p.y)};
+            m.e[7] = {T(p.z), T(p.w)};
+            m.e[8] = {T(q.x), T(q.y)};
         }
     } else {
 #pragma unroll
@@ -138,14 +160,26 @@ __device__ __forceinline__ void store_entries(vec2_t<S>* __restrict__ U, int64_t
 {
     const __amdgpu_buffer_rsrc_t r = planes_rsrc(U + (int64_t)mu * 9 * npad, npad, 9);
     if constexpr (sizeof(S) == 4) {
-        static_assert(K0 % 2 == 0 && (K1 % 2 == 0 || K1 == 9), "f32 links are written in pairs of entries");
-#pragma unroll
-        for (int k = K0; k + 1 < K1; k += 2)
-            buf_store<float4, CP>(r, link_off<S>(s, k), link_plane<S>(npad, k),
-                                  make_float4(S(m.e[k].re), S(m.e[k].im), S(m.e[k + 1].re), S(m.e[k + 1].im)));
-        if constexpr (K1 == 9)
+        static_assert((K0 == 0 || K0 == 6) && (K1 == 6 || K1 == 9), "f32 links are written in whole pairs");
+        const uint32_t off = link_off<S>(s, 0);
+        auto word = [&](int i, int j) __attribute__((always_inline)) {
+            return make_float4(S(m.e[i].re), S(m.e[i].im), S(m.e[j].re), S(m.e[j].im));
+        };
+        if constexpr (K0 == 0) {
+            buf_store<float4, CP>(r, off, link_plane<S>(npad, 0), word(0, 1));
+            buf_store<float4, CP>(r, off, link_plane<S>(npad, 2), word(3, 4));
+            float4 v = word(2, 5);
+            // opaque here: from the two halves of entries that are not neighbours
+            // the compiler makes overlapping vector reads of m, and m then
+            // stays in memory (k_drift 6.8 -> 20 us)
+            asm("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));
+            buf_store<float4, CP>(r, off, link_plane<S>(npad, 4), v);
+        }
+        if constexpr (K1 == 9) {
+            buf_store<float4, CP>(r, off, link_plane<S>(npad, 6), word(6, 7));
             buf_store<float2, CP>(r, link_off<S>(s, 8), link_plane<S>(npad, 8),
                                   make_float2(S(m.e[8].re), S(m.e[8].im)));
+        }
     } else {
 #pragma unroll
         for (int k = K0; k < K1; ++k)
