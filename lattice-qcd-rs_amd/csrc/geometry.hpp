@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "launch_order.hpp"
 #include "limits.hpp"
 
 namespace lqcd {
@@ -106,15 +107,13 @@ struct SiteCoords {
     }
 };
 
-// P and G of slab_block for workgroups of `block` sites, or 0 where the
-// lattice does not allow the order (whole workgroups per slice of the slowest
-// direction, 8 | its extent).
-inline void slab_shape(const Geom& g, int64_t block, int64_t& P, int64_t& G)
+// Site block of a workgroup in the order that P and G stand for
+// (launch_order.hpp).
+__device__ __forceinline__ int64_t ordered_block(int64_t P, int64_t G)
 {
-    const int64_t Ls = g.extent[g.dim - 1], slice = g.nsite / Ls;
-    const bool fits = slice % block == 0 && Ls % 8 == 0;
-    P = fits ? slice / block : 0;
-    G = fits ? Ls / 8 : 0;
+    if (P < 0) return blockIdx.x;
+    const int64_t b = xcd_remap(blockIdx.x, gridDim.x);
+    return P > 0 ? slab_block(b, P, G) : b;
 }
 
 template <int D>

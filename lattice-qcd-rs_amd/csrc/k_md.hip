@@ -43,15 +43,12 @@ namespace lqcd {
 // lanes' 8-byte writes fall into different banks) and the block stores the
 // image as whole 16-byte words, lane after lane.
 //
-// Bound by the neighbour links' latency (f64: one wave per SIMD, 440 VGPRs),
-// so the workgroups run in the MD kernels' order (xcd_remap, and slab_block
-// where the lattice allows it), which keeps neighbour blocks on one XCD.
-// Against storage order, same bits: f64 16^4 46.8 -> 37.0 us, 32^4 626 ->
-// 600, 15x13x11x17 32.9 -> 27.3, D = 3 128^3 745 -> 680; f32 24^4 141 -> 90,
-// 32^4 320 -> 300.  Workgroups of 64 or 256 threads, and f64 capped at two waves
+// Bound by the neighbour links' latency (f64: one wave per SIMD, 440 VGPRs);
+// the workgroups take the blocks in the order of force_order
+// (launch_order.hpp).  Workgroups of 64 or 256 threads, and f64 capped at two waves
 // per SIMD (spills 744 B; 16^4 70.6 us), were not faster.  Reading two rows of
-// SU(3) links is (16^4 30.6 us), but its error against 64 bits is 7 % (f64)
-// and 1 % (f32) larger, so all nine entries are read.
+// SU(3) links is (16^4 30.6 us against 37.0), but its error against 64 bits is 7 %
+// (f64) and 1 % (f32) larger, so all nine entries are read.
 constexpr int kForceBlock = 128;
 
 template <int D, typename S, typename T, bool PO>
@@ -61,9 +58,7 @@ __global__ __launch_bounds__(kForceBlock) void k_force_store(const vec2_t<S>* __
 {
     constexpr int kRow = D * 8 + 1;
     __shared__ double img[kForceBlock * kRow];
-    int64_t logical = xcd_remap(blockIdx.x, gridDim.x);
-    if (slab_p > 0) logical = slab_block(logical, slab_p, slab_g);
-    const int64_t s0 = logical * kForceBlock;
+    const int64_t s0 = ordered_block(slab_p, slab_g) * kForceBlock;
     const int64_t s = s0 + threadIdx.x;
     if (s < g.nsite) {
         const Neighbours<D> nb = neighbours<D>(g, s);
@@ -441,7 +436,7 @@ hipError_t launch_force_store(const lqcd_lattice* L, const void* U, double* d_ou
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_FORCE_STORE, &ev);
     int64_t slab_p, slab_g;
-    slab_shape(L->g, kForceBlock, slab_p, slab_g);
+    force_order(L->g, kForceBlock, slab_p, slab_g);
     const unsigned grid = grid_for(L->g.nsite, kForceBlock);
     LQCD_DISPATCH_DS_PO(L, k_force_store<D, S, S, PO><<<grid, kForceBlock, 0, L->ctx->stream>>>(
                                (const vec2_t<S>*)U, L->g, (S)md_force_scale(L->size), d_out, scale, slab_p, slab_g));

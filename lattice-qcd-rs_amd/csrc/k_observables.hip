@@ -10,31 +10,17 @@
 
 namespace lqcd {
 
-// The block of sites that a workgroup of the plaquette sums takes: neighbouring
-// blocks on one XCD (xcd_remap), in slabs where one pass of the grid covers the
-// lattice in whole slabs (slab_block); slab_p < 0: storage order.  The partials
-// keep the order of the
-// blocks, so the sums are the same bits in any order of the workgroups.
-__device__ __forceinline__ int64_t stencil_block(int64_t slab_p, int64_t slab_g)
-{
-    if (slab_p < 0) return blockIdx.x;
-    const int64_t b = xcd_remap(blockIdx.x, gridDim.x);
-    return slab_p > 0 ? slab_block(b, slab_p, slab_g) : b;
-}
-
 // plaquette_site summed over the lattice.  Bound by the neighbour links past the
-// L2; in the order of stencil_block against storage order: f32 32^4 160 ->
-// 120 us, 24^4 57.9 -> 42.6, 48^3 x 96 1726 -> 1608; f64 16^4 20.2 -> 17.0, 32^4 231 ->
-// 222.  D = 3 stays in storage order (128^3 f64 237 against 285 us): its
-// neighbours are two rows of one plane and two planes, which the eight L2s then
-// read together.
+// L2; the workgroups take the blocks in the order of plaquette_order
+// (launch_order.hpp).  The partials keep the order of the blocks, so the sums
+// are the same bits in any order of the workgroups.
 template <int D, typename S, bool PO>
 __global__ __launch_bounds__(kBlock) void k_plaquette_partials(const vec2_t<S>* __restrict__ U, Geom g,
                                                                double* __restrict__ partials, int64_t slab_p,
                                                                int64_t slab_g)
 {
     double acc[3] = {0.0, 0.0, 0.0};
-    const int64_t step = (int64_t)gridDim.x * kBlock, b = stencil_block(slab_p, slab_g);
+    const int64_t step = (int64_t)gridDim.x * kBlock, b = ordered_block(slab_p, slab_g);
     for (int64_t s = b * kBlock + threadIdx.x; s < g.nsite; s += step) plaquette_site<D, S, PO>(U, g, s, acc);
     block_reduce_to<3>(acc, partials + b * kReduceSlots);
 }
@@ -50,7 +36,7 @@ __global__ __launch_bounds__(kBlock) void k_hamiltonian_partials(const vec2_t<S>
                                                                  int64_t slab_g)
 {
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    const int64_t step = (int64_t)gridDim.x * kBlock, b = stencil_block(slab_p, slab_g);
+    const int64_t step = (int64_t)gridDim.x * kBlock, b = ordered_block(slab_p, slab_g);
     for (int64_t s = b * kBlock + threadIdx.x; s < g.nsite; s += step) {
 #pragma unroll
         for (int mu = 0; mu < D; ++mu) acc[3] += efield_energy_link<S>(E, g, mu, s);
@@ -144,20 +130,11 @@ static int reduce_blocks(int64_t n)
     return (int)b;
 }
 
-// slab order of the plaquette sums' nb workgroups, when they take one block
-// each (P < 0: storage order)
-static void sum_slabs(const lqcd_lattice* L, int nb, int64_t& P, int64_t& G)
-{
-    P = L->g.dim == 3 ? -1 : 0;
-    G = 0;
-    if (L->g.dim != 3 && (int64_t)nb * kBlock >= L->g.nsite) slab_shape(L->g, kBlock, P, G);
-}
-
 hipError_t launch_plaquette_sum(const lqcd_lattice* L, const void* U, double* d_out3)
 {
     const int nb = reduce_blocks(L->g.nsite);
     int64_t slab_p, slab_g;
-    sum_slabs(L, nb, slab_p, slab_g);
+    plaquette_order(L->g, slab_p, slab_g);
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_PLAQUETTE, &ev);
     LQCD_DISPATCH_DS_PO(L, k_plaquette_partials<D, S, PO><<<nb, kBlock, 0, L->ctx->stream>>>(
@@ -171,7 +148,7 @@ hipError_t launch_hamiltonian_sum(const lqcd_lattice* L, const void* U, const vo
 {
     const int nb = reduce_blocks(L->g.nsite);
     int64_t slab_p, slab_g;
-    sum_slabs(L, nb, slab_p, slab_g);
+    plaquette_order(L->g, slab_p, slab_g);
     lqcd_prof_event ev;
     prof_begin(L->ctx, PROF_PLAQUETTE, &ev);
     LQCD_DISPATCH_DS(L, k_hamiltonian_partials<D, S><<<nb, kBlock, 0, L->ctx->stream>>>(
