@@ -127,8 +127,16 @@ __device__ __forceinline__ int64_t class_site(const Geom& g, int64_t k, int pari
     return s0 + ((site_parity<D>(g, s0) + parity) & 1);
 }
 
-// Links of f64 lattices past the L2 are in parity order here (SiteMap, PO;
-// class_order_links in capi.cpp), others in site order.
+// The links of f64 lattices may be in parity order here (SiteMap, PO;
+// class_order_links in capi.cpp); others are in site order.
+//
+// Heat bath and overrelaxation store the new links evict-first: the next launch
+// reads another direction's class, and the L2 keeps the links of the staples.
+// 32^4 f32 heat bath 155 -> 149 us, overrelaxation 172 -> 168, 128^3 231 -> 223 and 273
+// -> 267; f64 in parity order 194 -> 192 and 210 -> 209, 288 -> 286 and 327 -> 322;
+// level on lattices whose links fit the 256 MB cache.  (With 16-byte words a
+// class load touches twice the lines of a word per entry, half used, and the f32
+// launches fetched 11 % more past the L2: 145 and 164 us at 32^4 with the latter.)
 //
 // Order of a class launch's workgroups: each covers 2 kBlock consecutive
 // sites (kBlock class links); XCD k gets a contiguous range of them
@@ -396,7 +404,7 @@ __global__ __launch_bounds__(kBlock) void k_heat_bath(vec2_t<S>* __restrict__ U,
     }
     mat3<double> nw;
     mul<false, false>(acc, u, nw);
-    store_link<double, S>(U, g.npad, mu, own, nw);
+    store_link<double, S, kCacheStream>(U, g.npad, mu, own, nw);
     const int64_t o = (int64_t)(mu * 2 + parity) * (g.nsite / 2) + k;
     p_out[o] = 0.0;
     exhausted[o] = ex;
@@ -558,7 +566,7 @@ __global__ __launch_bounds__(kBlock) void k_overrelax(vec2_t<S>* __restrict__ U,
         mul<false, true>(rot, u, t);
         mul<false, false>(t, rot, nw);
     }
-    store_link<double, S>(U, g.npad, mu, own, nw);
+    store_link<double, S, kCacheStream>(U, g.npad, mu, own, nw);
 }
 
 // Links in site order -> parity order (TO_PARITY) or back, one link per thread
