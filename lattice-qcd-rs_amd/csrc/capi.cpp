@@ -1123,12 +1123,13 @@ int lqcd_wilson_backward_device(lqcd_lattice* L, double beta, double* d_grad, si
 // The order of the links for a sweep.  A class updates the sites of one
 // parity, every other one of a row: in site order its loads use half of each
 // 128-byte line, and the other half comes in again for the next staple.  In
-// parity order f64 class launches take, at 32^4: heat bath 328 -> 204 us,
-// overrelaxation 325 -> 241, Metropolis 200 -> 137; D = 3 128^3: 442 -> 295,
-// 455 -> 377, 271 -> 209.  Sweeps, link updates, normalisation, plaquette and force read
-// either order (the last two up to 19 % slower in parity order: 32^4 212 ->
-// 246 and 561 -> 604 us); other calls turn it back (site_order_links).  When
-// that pays: sweep_order.hpp.  LQCD_SWEEP_ORDER=site or parity (f64 fields of
+// parity order class launches take, at 32^4: f64 heat bath 328 -> 194 us,
+// overrelaxation 319 -> 209, Metropolis 198 -> 137, f32 150 -> 123 and 168 ->
+// 150; D = 3 128^3 f64: 362 -> 218 (heat bath), 361 -> 246, 208 -> 158.  Sweeps, link
+// updates, normalisation, plaquette and force read either order (the last two
+// up to 19 % slower in parity order, 25 % in f32: 32^4 f64 212 -> 246 and 561 -> 604
+// us); other calls turn it back (site_order_links).  When that pays:
+// sweep_order.hpp.  LQCD_SWEEP_ORDER=site or parity (where it is built, fields of
 // any size) pins the order.
 static int class_order_links(lqcd_lattice* L, SweepKind kind, size_t n_update)
 {
@@ -1141,7 +1142,7 @@ static int class_order_links(lqcd_lattice* L, SweepKind kind, size_t n_update)
             HIP_TRY(site_order_links(L));
             return LQCD_OK;
         }
-        if (std::strcmp(env, "parity") == 0) parity = L->precision == LQCD_F64;
+        if (std::strcmp(env, "parity") == 0) parity = parity_order_built(L->precision == LQCD_F64, L->g.dim);
     }
     if (L->parity_order || !parity) return LQCD_OK;
     const int w = (L->cur + 1) % 3;

@@ -33,19 +33,25 @@
         }                                                                           \
     } while (0)
 
-// as LQCD_DISPATCH_DS, with PO: the lattice's links are in parity order (f64
-// storage only)
+// as LQCD_DISPATCH_DS, with PO: the lattice's links are in parity order
+// (parity_order_built)
 #define LQCD_DISPATCH_DS_PO(L, ...)                                                 \
     do {                                                                            \
         if ((L)->parity_order) {                                                    \
             constexpr bool PO = true;                                               \
-            using S = double;                                                       \
-            if ((L)->precision != 0) return hipErrorInvalidValue;                   \
-            switch ((L)->g.dim) {                                                   \
-            case 2: { constexpr int D = 2; __VA_ARGS__; } break;                    \
-            case 3: { constexpr int D = 3; __VA_ARGS__; } break;                    \
-            case 4: { constexpr int D = 4; __VA_ARGS__; } break;                    \
-            default: return hipErrorInvalidValue;                                   \
+            if ((L)->precision == 0) {                                              \
+                using S = double;                                                   \
+                switch ((L)->g.dim) {                                               \
+                case 2: { constexpr int D = 2; __VA_ARGS__; } break;                \
+                case 3: { constexpr int D = 3; __VA_ARGS__; } break;                \
+                case 4: { constexpr int D = 4; __VA_ARGS__; } break;                \
+                default: return hipErrorInvalidValue;                               \
+                }                                                                   \
+            } else {                                                                \
+                using S = float;                                                    \
+                constexpr int D = 4;                                                \
+                if ((L)->g.dim != D) return hipErrorInvalidValue;                   \
+                __VA_ARGS__;                                                        \
             }                                                                       \
         } else {                                                                    \
             constexpr bool PO = false;                                              \

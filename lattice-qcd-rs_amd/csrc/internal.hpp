@@ -39,7 +39,7 @@ struct lqcd_lattice {
     void* U[3] = {nullptr, nullptr, nullptr};
     int cur = 0;             // buffer holding the current links
     // the current links are in parity order (SiteMap in geometry.hpp): set by
-    // the f64 checkerboard sweeps, undone by site_order_links before anything
+    // the checkerboard sweeps, undone by site_order_links before anything
     // that reads them in site order
     bool parity_order = false;
     lqcd::SweepOrder order;  // when they are put there

@@ -127,8 +127,8 @@ __device__ __forceinline__ int64_t class_site(const Geom& g, int64_t k, int pari
     return s0 + ((site_parity<D>(g, s0) + parity) & 1);
 }
 
-// The links of f64 lattices may be in parity order here (SiteMap, PO;
-// class_order_links in capi.cpp); others are in site order.
+// The links may be in parity order here (SiteMap, PO;
+// class_order_links in capi.cpp).
 //
 // Heat bath and overrelaxation store the new links evict-first: the next launch
 // reads another direction's class, and the L2 keeps the links of the staples.

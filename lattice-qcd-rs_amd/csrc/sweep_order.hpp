@@ -10,7 +10,7 @@ enum SweepKind { SWEEP_METROPOLIS, SWEEP_HEAT_BATH, SWEEP_OVERRELAX };
 
 // What a sweep gains in parity order, in units of the two reorderings that it
 // costs to go there and back; 0: not worth it.  The least that was measured
-// (us per sweep and per two reorderings, f64, site -> parity order):
+// (us per sweep and per two reorderings, site -> parity order, f64 first):
 //                two     Metropolis,   Metropolis,    heat bath     overrelaxation
 //                        1 update      10 updates                   (either kind: the lesser gain)
 //   16^4          31      197 ->  188   396 ->  384    281 ->  247    314 ->  281
@@ -25,13 +25,24 @@ enum SweepKind { SWEEP_METROPOLIS, SWEEP_HEAT_BATH, SWEEP_OVERRELAX };
 //   342^2         29      102 ->   97   202 ->  204    137 ->  131    158 ->  151
 //   512^2         56      151 ->  130   344 ->  316    222 ->  184    510 ->  474
 //   2048^2       939     1631 -> 1216  3726 -> 3730   2391 -> 1551   2452 -> 2190
-// Links that fit in the 32 MiB of the eight L2s stay in site order, and f32
-// links, where a class launch gains 6-11 %, less than two reorderings cost.
+//   f32:
+//   20^4          37      277 ->  268   650 ->  633    370 ->  335    428 ->  401
+//   24^4          67      353 ->  343   888 ->  874    532 ->  455    629 ->  538
+//   32^4         221      730 ->  683  2122 -> 2077   1199 ->  986   1362 -> 1197
+//   40^4         503     1935 -> 1783  5258 -> 5151   2791 -> 2334   3177 -> 2866
+//   128^3        343      938 ->  899  2950 -> 3042   1329 -> 1235   1628 -> 1580
+// Links that fit in the 32 MiB of the eight L2s stay in site order.  In f32 only
+// the heat bath and overrelaxation of D = 4 gain more than plaquette, force and
+// normalisation lose in this order (32^4 113 -> 141, 275 -> 306, 78 -> 88 us).
 constexpr size_t kParityOrderBytes = (size_t)32 << 20;
+
+// whether the kernels read links in parity order (LQCD_DISPATCH_DS_PO)
+inline bool parity_order_built(bool f64, int dim) { return f64 || dim == 4; }
 
 inline double parity_order_gain(SweepKind kind, bool f64, int dim, size_t link_bytes, size_t n_update)
 {
-    if (!f64 || link_bytes < kParityOrderBytes) return 0.0;
+    if (link_bytes < kParityOrderBytes) return 0.0;
+    if (!f64) return dim == 4 && kind != SWEEP_METROPOLIS ? 0.6 : 0.0;
     const bool large = link_bytes >= 2 * kParityOrderBytes;
     if (kind != SWEEP_METROPOLIS) {
         if (dim == 4) return large ? 1.3 : 1.0;
